@@ -69,6 +69,9 @@ static std::map<std::string, int64_t> g_tune = {
     // without deferral); read when an SSSP handle is created
     {"sssp_delta", 0},
     {"sssp_far_cap", 0},  // entries per near-far list (0: one per vertex)
+    // static triangle count: most scratch for its sorted lists, in MB (0: no
+    // bound); a graph that needs more is counted over its plain lists
+    {"tc_scratch_mb", 0},
 };
 
 int64_t tune_get(const char *name, int64_t dflt) {
@@ -690,6 +693,8 @@ int mk_tune_set(const char *name, int64_t value) {
   if (k == "pull_exit" && value == 0) return fail(MK_ERR_BAD_ARG, "pull_exit must be >= 1");
   if (k == "sssp_far_cap" && (value < 0 || value > 0xFFFFFFF0ll))
     return fail(MK_ERR_BAD_ARG, "sssp_far_cap must be in [0, 4294967280]");
+  if (k == "tc_scratch_mb" && (value < 0 || value > (1 << 24)))
+    return fail(MK_ERR_BAD_ARG, "tc_scratch_mb must be in [0, 16777216]");
   if (k == "sssp_delta" && (value < 0 || value > (1 << 24)))
     return fail(MK_ERR_BAD_ARG, "sssp_delta must be in [0, 16777216]");
   std::lock_guard<std::mutex> lk(g_tune_mu);

@@ -9,12 +9,15 @@
 //
 // Method here (same counts):
 //  - Static: vertices are ranked by (degree, id) and N+(x) holds the
-//    neighbours of x ranked above x (|N+(x)| <= sqrt(2m)).  Each triangle
-//    a < b < c is counted once, at a, as an element of N+(a) and N+(b) for b
-//    in N+(a).  The N+ lists are built compactly in HBM (count pass,
-//    exclusive scan, fill pass over the slabs); then one wave per vertex a
-//    puts N+(a) (1024 keys at a time) into an LDS hash table and streams
-//    every N+(b), b in N+(a), through it with coalesced loads.
+//    neighbours of x ranked above x (|N+(x)| <= sqrt(2m)), as ranks, sorted.
+//    Each triangle a < b < c is counted once, at b: as a c past b in N+(a),
+//    for an a with b in N+(a), that is in N+(b) too.  Every vertex b has the
+//    list of its (a, place of b in N+(a)); a wave puts N+(b) into LDS and
+//    tests the tails of those N+(a) against it, so that every wedge is
+//    looked at once (see "wedges" below).  Where the device memory for
+//    these lists (16 bytes per undirected edge) is short, the N+ lists
+//    alone (4 bytes) are built, a wave per vertex a puts N+(a) into an LDS
+//    hash table and every N+(b) is streamed through it.
 //  - Incremental / Decremental: the batch's changed undirected edges (the
 //    entries the last insert / delete applied) go into a device hash set.
 //    For each changed edge {u, v} the wave enumerates the neighbours w of the
@@ -28,6 +31,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <numeric>
 
 #include "profile.hpp"
 #include "slabhash.hpp"
@@ -281,6 +285,371 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
+// ---------------------------------------------------------------- wedges
+// The static count over sorted lists of ranks.  RMAT-20 (15.7M undirected
+// edges): the tails tested are 1.23e9 elements, where streaming every N+(b)
+// against N+(a) reads 4.42e9.
+constexpr uint32_t kTableWords = 1024;  // LDS words per wave: bitmap or hash table
+constexpr uint32_t kTopRanks = kTableWords * 32;  // highest ranks a bitmap covers exactly
+constexpr uint32_t kUnit = 64;          // list entries per unit of k_tc_wedges
+constexpr uint32_t kTakers = 16;         // unit counters
+constexpr uint32_t kSortRow = 1024;     // row elements staged in LDS at a time
+constexpr uint32_t kTail = 8;           // lanes per tail
+constexpr uint32_t kRounds = 4;         // elements a lane takes at a time
+
+// Orders the wave's LDS accesses before and after it (the LDS unit takes a
+// wave's accesses in order: no instruction, the compiler only).
+MK_DEV void lds_settle() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__global__ void k_tc_iota(uint32_t *p, uint32_t n) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = i;
+}
+
+// rank[order[i]] = i; row i (a rank) starts with room for its whole degree.
+__global__ void k_tc_rank(const uint32_t *order, const uint32_t *sdeg, uint32_t n, uint32_t *rank,
+                          unsigned long long *deg) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  rank[order[i]] = i;
+  deg[i] = sdeg[i];
+}
+
+// One pass over the slabs, an 8-lane group per bucket: the ranks above the
+// owner's, appended to the owner's row (`cursor`: one atomic per slab).
+// Rows have room for the whole degree, so nothing is counted first.  Bound
+// by the rank gathers (one per key, from an array of 4 bytes a vertex).
+template <bool MAP>
+__global__ void __launch_bounds__(kBlock)
+    k_tc_rows(GraphView G, const uint32_t *rank, const unsigned long long *row0, uint32_t *len,
+              uint32_t *raw, unsigned long long *slab_count) {
+  const uint32_t gl = group_lane();
+  const uint64_t g0 = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kGroupLanes;
+  const uint64_t NG = uint64_t(gridDim.x) * blockDim.x / kGroupLanes;
+  uint32_t slabs = 0;
+  for (uint64_t b = g0; b < G.total_buckets; b += NG) {
+    const uint32_t u = G.bucket_owner[b];
+    if (G.vdeg[u] == 0) continue;
+    const uint32_t r = rank[u];
+    const uint32_t *slab = G.heads + b * kSlabWords;
+    for (;;) {
+      ++slabs;
+      uint32_t x[kWordsPerLane], rx[kWordsPerLane];
+      load_words(slab + kWordsPerLane * gl, x);
+      uint32_t c = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < kWordsPerLane; ++k)
+        rx[k] = key_word<MAP>(kWordsPerLane * gl + k) && x[k] < kTomb ? rank[x[k]] : 0u;
+#pragma unroll
+      for (uint32_t k = 0; k < kWordsPerLane; ++k) c += rx[k] > r ? 1u : 0u;
+      uint32_t pre = c;  // inclusive over the group
+#pragma unroll
+      for (uint32_t o = 1; o < kGroupLanes; o <<= 1) {
+        const uint32_t y = uint32_t(__shfl_up(int(pre), o, int(kGroupLanes)));
+        if (gl >= o) pre += y;
+      }
+      const uint32_t sum = group_read(pre, kGroupLanes - 1);
+      if (sum) {
+        uint32_t at = 0;
+        if (gl == 0) at = atomicAdd(len + r, sum);
+        unsigned long long pos = row0[r] + group_read(at, 0) + (pre - c);
+#pragma unroll
+        for (uint32_t k = 0; k < kWordsPerLane; ++k)
+          if (rx[k] > r) raw[pos++] = rx[k];
+      }
+      const uint32_t nx = group_read(x[kWordsPerLane - 1], kGroupLanes - 1);
+      if (nx == kEmpty) break;
+      slab = slab_ptr(G.pool, nx);
+    }
+  }
+  slabs = wave_sum_u32(gl == 0 ? slabs : 0u);
+  if (lane_id() == 0 && slabs) atomicAdd(slab_count, (unsigned long long)slabs);
+}
+
+// Where vertex b's list counter lies: neighbouring ranks, all hubs at the
+// top, are kSpread columns apart, so that their counters share no line
+// (atomics on one line follow one another: RMAT-20's counts took 2.6 ms in
+// rank order).
+constexpr uint32_t kSpread = 1024;
+__host__ __device__ inline uint32_t spread_rows(uint32_t n) { return (n + kSpread - 1) / kSpread; }
+MK_DEV uint32_t spread_index(uint32_t b, uint32_t n) {
+  return (b % kSpread) * spread_rows(n) + b / kSpread;
+}
+
+// Row (or spread list) lengths as 64-bit values with a zero behind them.
+__global__ void k_tc_widen(const uint32_t *len, uint32_t n, bool spread, unsigned long long *out) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= n) out[i] = i < n ? len[spread ? spread_index(i, n) : i] : 0ull;
+}
+
+// Sort every row (ranks are distinct: an element's place is the number of
+// smaller ones) into `up`, and give every element b but a row's last, whose
+// tail is empty, its place in b's list: slot[e] = entries of b so far
+// (kEmpty: none, also when N+(b) is empty).  A wave takes 64 rows: single
+// elements lane by lane, rows of up to 64 in registers, longer ones staged
+// in LDS kSortRow at a time.
+MK_DEV uint32_t tc_slot(uint32_t b, bool tail, const uint32_t *len, uint32_t *ndown, uint32_t n) {
+  return tail && len[b] ? atomicAdd(ndown + spread_index(b, n), 1u) : kEmpty;
+}
+__global__ void __launch_bounds__(kBlock)
+    k_tc_sort(const unsigned long long *row0, const uint32_t *len, const unsigned long long *off,
+              const uint32_t *raw, uint32_t n, uint32_t *up, uint32_t *slot, uint32_t *ndown) {
+  __shared__ uint32_t stage[kBlock / 64][kSortRow];
+  const uint32_t lane = lane_id();
+  uint32_t *st = stage[threadIdx.x >> 6];
+  const uint64_t gw = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
+  const uint64_t W = (uint64_t(gridDim.x) * blockDim.x) >> 6;
+  for (uint64_t r0 = gw; r0 * 64 < n; r0 += W) {
+    // lane i: row i * ceil(n / 64) + r0, so that a wave's rows are spread
+    // over the ranks (long rows are neighbours)
+    const uint64_t r = uint64_t(lane) * ((uint64_t(n) + 63) / 64) + r0;
+    const bool mine = r < n && r0 < (uint64_t(n) + 63) / 64;
+    const uint32_t K = mine ? len[r] : 0u;
+    const unsigned long long src = mine ? row0[r] : 0ull, dst = mine ? off[r] : 0ull;
+    if (K == 1) {
+      up[dst] = raw[src];
+      slot[dst] = kEmpty;
+    }
+    uint64_t m = ballot(K > 1);
+    while (m) {
+      const uint32_t j = ffs64(m);
+      m &= m - 1;
+      const uint32_t k = read_lane(K, j);
+      const uint32_t *in = raw + (uint64_t(read_lane(uint32_t(src >> 32), j)) << 32 |
+                                  read_lane(uint32_t(src), j));
+      const unsigned long long o = uint64_t(read_lane(uint32_t(dst >> 32), j)) << 32 |
+                                   read_lane(uint32_t(dst), j);
+      if (k <= 64) {
+        const uint32_t x = lane < k ? in[lane] : kEmpty;
+        uint32_t at = 0;
+        for (uint32_t i = 0; i < k; ++i) at += read_lane(x, i) < x ? 1u : 0u;
+        if (lane < k) {
+          up[o + at] = x;
+          slot[o + at] = tc_slot(x, at + 1 < k, len, ndown, n);
+        }
+        continue;
+      }
+      for (uint32_t c0 = 0; c0 < k; c0 += 64) {
+        const uint32_t x = c0 + lane < k ? in[c0 + lane] : kEmpty;
+        uint32_t at = 0;
+        for (uint32_t t0 = 0; t0 < k; t0 += kSortRow) {
+          const uint32_t tn = min(kSortRow, k - t0);
+          if (c0 == 0 || k > kSortRow) {  // one tile: staged once
+            lds_settle();
+            for (uint32_t i = lane; i < (tn + 3) / 4 * 4; i += 64)
+              st[i] = i < tn ? in[t0 + i] : kEmpty;
+            lds_settle();
+          }
+          for (uint32_t i = 0; i < tn; i += 4) {
+            const uint4 y = *reinterpret_cast<const uint4 *>(st + i);
+            at += (y.x < x ? 1u : 0u) + (y.y < x ? 1u : 0u) + (y.z < x ? 1u : 0u) +
+                  (y.w < x ? 1u : 0u);
+          }
+        }
+        if (c0 + lane < k) {
+          up[o + at] = x;
+          slot[o + at] = tc_slot(x, at + 1 < k, len, ndown, n);
+        }
+      }
+      lds_settle();
+    }
+  }
+}
+
+// Entry of b's list: the tail of a row past b, (first element << 24) | length.
+// Rows shorter than 2^24 (their square is at most 2 m).  Eight rows to a
+// wave: neighbouring ranks' rows are long together (64 to a wave left the
+// last waves running for 0.9 ms on RMAT-20).
+constexpr uint32_t kDownRows = 8;
+__global__ void __launch_bounds__(kBlock)
+    k_tc_down(const uint32_t *len, const unsigned long long *off, const uint32_t *up,
+              const uint32_t *slot, const unsigned long long *doff, uint32_t n,
+              unsigned long long *down) {
+  const uint32_t lane = lane_id();
+  const uint64_t gw = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
+  const uint64_t W = (uint64_t(gridDim.x) * blockDim.x) >> 6;
+  for (uint64_t r0 = gw * kDownRows; r0 < n; r0 += W * kDownRows) {
+    // the rows' elements together, 64 at a time
+    const uint32_t K = lane < kDownRows && r0 + lane < n ? len[r0 + lane] : 0u;
+    uint32_t incl = K;
+#pragma unroll
+    for (uint32_t o = 1; o < kDownRows; o <<= 1) {
+      const uint32_t y = uint32_t(__shfl_up(int(incl), o, 64));
+      if (lane >= o) incl += y;
+    }
+    const uint32_t total = read_lane(incl, kDownRows - 1);
+    const unsigned long long base = off[r0];
+    for (uint32_t e = lane; e < total; e += 64) {
+      uint32_t end = total;  // the end of e's row
+#pragma unroll
+      for (uint32_t k = kDownRows - 1; k > 0; --k) {
+        const uint32_t x = read_lane(incl, k - 1);
+        if (e < x) end = x;
+      }
+      const uint32_t s = slot[base + e];
+      if (s != kEmpty) down[doff[up[base + e]] + s] = ((base + e + 1) << 24) | (end - e - 1);
+    }
+  }
+}
+
+// The vertex whose list holds the first entry of every unit.
+__global__ void k_tc_units(const unsigned long long *doff, uint32_t n, uint32_t *unit_b) {
+  const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= n) return;
+  for (unsigned long long u = (doff[b] + kUnit - 1) / kUnit; u * kUnit < doff[b + 1]; ++u)
+    unit_b[u] = b;
+}
+
+MK_DEV uint32_t table_slot(uint32_t x) {
+  static_assert(kTableWords == 1u << 10, "ten hash bits");
+  return (x * 2654435761u) >> (32 - 10);
+}
+
+// The wedges of one run of entries [s, e) of vertex b against N+(b) in the
+// wave's table.  Each 8-lane group takes every eighth entry, 32 elements of
+// its tail at a time, the next 32 in flight; groups go on to their next
+// entry independently.  BITS: exact bitmap of the ranks from `top` on; else an
+// open-addressing hash table.
+template <bool BITS>
+MK_DEV void tc_tails(const uint32_t *tab, uint32_t top, const unsigned long long *down,
+                     unsigned long long s, unsigned long long e, const uint32_t *up,
+                     uint64_t &count) {
+  const uint32_t gl = lane_id() & (kTail - 1);
+  unsigned long long i = s + lane_id() / kTail;
+  unsigned long long ent = i < e ? down[i] : 0ull;
+  i += 64 / kTail;
+  unsigned long long nxt = i < e ? down[i] : 0ull;
+  unsigned long long p = ent >> 24, end = p + (ent & 0xFFFFFFull);
+  uint32_t hits = 0;
+  uint32_t c[kRounds], d[kRounds];  // this round's elements and the next one's, in flight
+#pragma unroll
+  for (uint32_t k = 0; k < kRounds; ++k) {
+    const unsigned long long q = p + k * kTail + gl;
+    d[k] = q < end ? up[q] : kEmpty;
+  }
+  bool more = ballot(p < end) != 0;
+  while (more) {
+    p += kRounds * kTail;
+    if (p >= end) {  // the group's next entry (0: none, an empty tail)
+      p = nxt >> 24;
+      end = p + (nxt & 0xFFFFFFull);
+      i += 64 / kTail;
+      nxt = i < e ? down[i] : 0ull;
+    }
+    more = ballot(p < end) != 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kRounds; ++k) {
+      c[k] = d[k];
+      const unsigned long long q = p + k * kTail + gl;
+      d[k] = q < end ? up[q] : kEmpty;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kRounds; ++k) {
+      if (c[k] == kEmpty) continue;
+      if (BITS) {
+        const uint32_t x = c[k] - top;
+        hits += (tab[x >> 5] >> (x & 31u)) & 1u;
+      } else {
+        uint32_t sl = table_slot(c[k]);
+        for (;;) {
+          const uint32_t t = tab[sl];
+          if (t == c[k]) {
+            ++hits;
+            break;
+          }
+          if (t == kEmpty) break;
+          sl = (sl + 1) & (kTableWords - 1);
+        }
+      }
+    }
+  }
+  count += hits;
+}
+
+// The wedge count: a wave per unit of kUnit consecutive list entries (units
+// in a permuted order: neighbours cost alike), vertex after vertex of the
+// unit.  N+(b) goes into the wave's table: for the kTopRanks highest ranks
+// a bitmap (every element is ranked above b, so the table is exact; one LDS
+// read a test), below them a hash table of up to kTableWords / 2 elements at
+// a time.  Bound by the latency of the tails' loads, so the table is small
+// enough for 32 waves a CU: RMAT-20's 1.23e9 tests take 1.10 ms, 1.83 ms at
+// 2048 words (20 waves a CU); units of 256 entries took as long there, but
+// 2.4x at RMAT-17, whose last units ran alone; 16 lanes a tail 1.17 ms.
+__global__ void __launch_bounds__(kBlock)
+    k_tc_wedges(const uint32_t *len, const unsigned long long *off, const uint32_t *up,
+                const unsigned long long *doff, const unsigned long long *down,
+                const uint32_t *unit_b, uint32_t n, uint64_t entries, uint64_t units,
+                uint64_t stride, unsigned long long *next, unsigned long long *slots) {
+  __shared__ uint32_t table[kBlock / 64][kTableWords];
+  uint32_t *tab = table[threadIdx.x >> 6];
+  const uint32_t lane = lane_id();
+  const uint64_t gw = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
+  const uint32_t top = n > kTopRanks ? n - kTopRanks : 0u;
+  uint64_t count = 0;
+  // waves take units from kTakers counters (a line each) that share the
+  // units out between them: one counter would hand out a unit every 11 ns
+  const uint32_t taker = uint32_t(gw % kTakers);
+  for (;;) {
+    unsigned long long t = 0;
+    if (lane == 0) t = atomicAdd(next + taker * 16, 1ull);
+    const uint64_t k =
+        (uint64_t(read_lane(uint32_t(t >> 32), 0)) << 32 | read_lane(uint32_t(t), 0)) * kTakers +
+        taker;
+    if (k >= units) break;
+    const uint64_t p0 = (k * stride % units) * kUnit, p1 = min(p0 + kUnit, entries);
+    for (uint32_t b0 = unit_b[p0 / kUnit]; b0 < n; b0 += 64) {
+      // 64 vertices' lists at once: those with entries in this unit
+      const uint32_t bl = b0 + lane;
+      const unsigned long long d0 = bl < n ? doff[bl] : entries;
+      const unsigned long long d1 = bl < n ? doff[bl + 1] : entries;
+      uint64_t m = ballot(d0 < d1 && d0 < p1 && d1 > p0);
+      const bool last = ballot(d1 >= p1) != 0;
+      while (m) {
+        const uint32_t j = ffs64(m);
+        m &= m - 1;
+        const uint32_t b = b0 + j;
+        const unsigned long long s = max<uint64_t>(doff[b], p0), e = min<uint64_t>(doff[b + 1], p1);
+        const uint32_t K = len[b];
+        const uint32_t *row = up + off[b];
+        if (b >= top) {
+          lds_settle();
+          for (uint32_t i = lane * 4; i < kTableWords; i += 256)
+            *reinterpret_cast<uint4 *>(tab + i) = make_uint4(0u, 0u, 0u, 0u);
+          lds_settle();
+          for (uint32_t i = lane; i < K; i += 64) {
+            const uint32_t x = row[i] - top;
+            atomicOr(tab + (x >> 5), 1u << (x & 31u));
+          }
+          lds_settle();
+          tc_tails<true>(tab, top, down, s, e, up, count);
+        } else {
+          for (uint32_t c0 = 0; c0 < K; c0 += kTableWords / 2) {
+            const uint32_t cn = min(kTableWords / 2, K - c0);
+            lds_settle();
+            for (uint32_t i = lane * 4; i < kTableWords; i += 256)
+              *reinterpret_cast<uint4 *>(tab + i) = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
+            lds_settle();
+            for (uint32_t i = lane; i < cn; i += 64) {
+              const uint32_t x = row[c0 + i];
+              uint32_t sl = table_slot(x);
+              while (atomicCAS(tab + sl, kEmpty, x) != kEmpty) sl = (sl + 1) & (kTableWords - 1);
+            }
+            lds_settle();
+            tc_tails<false>(tab, 0u, down, s, e, up, count);
+          }
+        }
+      }
+      if (last) break;
+    }
+  }
+  count = wave_sum_u64(count);
+  if (lane == 0) add_count(slots, count);
+}
+
 // Canonical changed edges of a batch: entries with status == APPLIED (or all
 // non-loop entries when status is NULL) enter the set; the first entry of
 // each undirected edge appends it to `owned`.
@@ -455,6 +824,7 @@ struct TC {
   unsigned long long *slots = nullptr;
   uint32_t *n_owned = nullptr;
   DevBuf tab, owned, ddeg, doff, cursor, dlist, scan_tmp, kup, koff, uplist, grabs;
+  DevBuf ranks, rows, raw, slot, units;  // static count over sorted rows
   HostBuf host;
   unsigned long long count = 0;
   uint64_t last_slabs = 0, last_streamed = 0;
@@ -480,7 +850,8 @@ struct TC {
     (void)hipFree(slots);
     (void)hipFree(n_owned);
     for (DevBuf *b :
-         {&tab, &owned, &ddeg, &doff, &cursor, &dlist, &scan_tmp, &kup, &koff, &uplist, &grabs})
+         {&tab, &owned, &ddeg, &doff, &cursor, &dlist, &scan_tmp, &kup, &koff, &uplist, &grabs,
+          &ranks, &rows, &raw, &slot, &units})
       b->release();
     host.release();
     if (ev0) (void)hipEventDestroy(ev0);
@@ -515,8 +886,133 @@ struct TC {
     return MK_OK;
   }
 
+  // hipcub exclusive sum of n + 1 values on the handle's stream.
+  int exclusive_sum(const unsigned long long *in, unsigned long long *out) {
+    const int items = int(size_t(g->n) + 1);
+    size_t tmp = 0;
+    MK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, in, out, items, stream));
+    if (int r = scan_tmp.ensure(tmp)) return r;
+    MK_HIP(hipcub::DeviceScan::ExclusiveSum(scan_tmp.ptr, tmp, in, out, items, stream));
+    return MK_OK;
+  }
+  int read_word(const unsigned long long *p, uint64_t &x) {
+    MK_HIP(hipMemcpyAsync(host.ptr, p, 8, hipMemcpyDeviceToHost, stream));
+    MK_HIP(hipStreamSynchronize(stream));
+    x = *host.as<uint64_t>();
+    return MK_OK;
+  }
+  // Grow a buffer with an eighth to spare; false when memory is short.
+  static bool fits(DevBuf &b, uint64_t bytes) {
+    if (b.ptr && b.bytes >= bytes) return true;
+    if (b.ensure(bytes + bytes / 8) == MK_OK || b.ensure(bytes) == MK_OK) return true;
+    (void)hipGetLastError();
+    return false;
+  }
+
+  // The wedge count queued on the stream (its result in `slots`), or
+  // *done = false when device memory for its lists is short (or over the
+  // knob "tc_scratch_mb"): nothing is counted then.
+  int queue_wedges(bool *done) {
+    *done = false;
+    const uint32_t n = g->n;
+    const uint64_t limit = uint64_t(tune_get("tc_scratch_mb", 0)) << 20;
+    // ranks: keys and values of the sort by (degree, id), both ways, and
+    // the rank of each vertex; rows: places and lengths
+    const size_t n1 = size_t(spread_rows(n)) * kSpread + 2;
+    if (!fits(ranks, n1 * 16) || !fits(rows, n1 * 32)) return MK_OK;
+    uint32_t *rank = ranks.as<uint32_t>(), *ids = rank + n1, *order = ids + n1, *sdeg = order + n1;
+    unsigned long long *row0 = rows.as<unsigned long long>(), *off = row0 + n1, *tmp = off + n1;
+    uint32_t *len = reinterpret_cast<uint32_t *>(tmp + n1), *ndown = len + n1;
+    const unsigned tgrid = blocks_for_threads(n), grid = blocks_for_waves(
+        std::min<uint64_t>((uint64_t(n) + 7) / 8, uint64_t(device_cus(g->device)) * 32));
+    ProfScope prof(stream, "k_tc_lists", 0.0);
+    k_tc_iota<<<tgrid, kBlock, 0, stream>>>(ids, n);
+    // degrees are below n (no self-loops, no duplicates)
+    int bits = 1;
+    while (bits < 32 && (n >> bits)) ++bits;
+    size_t need = 0;
+    MK_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, need, g->vdeg, sdeg, ids, order, int(n), 0,
+                                              bits, stream));
+    if (!fits(scan_tmp, need)) return MK_OK;
+    MK_HIP(hipcub::DeviceRadixSort::SortPairs(scan_tmp.ptr, need, g->vdeg, sdeg, ids, order,
+                                              int(n), 0, bits, stream));
+    fill_u64(reinterpret_cast<uint64_t *>(tmp) + n, 0ull, 1, stream);
+    k_tc_rank<<<tgrid, kBlock, 0, stream>>>(order, sdeg, n, rank, tmp);
+    if (int r = exclusive_sum(tmp, row0)) return r;
+    uint64_t total = 0;
+    if (int r = read_word(row0 + n, total)) return r;
+    if (limit && total * 8 > limit) return MK_OK;  // 4 B here and 4 B below a direction
+    if (!fits(raw, std::max<uint64_t>(total, 1) * 4)) return MK_OK;
+    fill_u32(len, 0u, 2 * n1, stream);  // and ndown
+    const unsigned bgrid = blocks_for_waves(std::min<uint64_t>(
+        (uint64_t(g->total_buckets) + 7) / 8, uint64_t(device_cus(g->device)) * 32));
+    auto kr = g->weighted ? k_tc_rows<true> : k_tc_rows<false>;
+    kr<<<bgrid, kBlock, 0, stream>>>(g->view(), rank, row0, len, raw.as<uint32_t>(),
+                                     slots + kTcSlots);
+    k_tc_widen<<<blocks_for_threads(uint64_t(n) + 1), kBlock, 0, stream>>>(len, n, false, tmp);
+    if (int r = exclusive_sum(tmp, off)) return r;
+    uint64_t ups = 0;
+    if (int r = read_word(off + n, ups)) return r;
+    if (ups == 0) {
+      *done = true;
+      return MK_OK;
+    }
+    if (!fits(uplist, ups * 4) || !fits(slot, ups * 4)) return MK_OK;
+    k_tc_sort<<<grid, kBlock, 0, stream>>>(row0, len, off, raw.as<uint32_t>(), n,
+                                           uplist.as<uint32_t>(), slot.as<uint32_t>(), ndown);
+    k_tc_widen<<<blocks_for_threads(uint64_t(n) + 1), kBlock, 0, stream>>>(ndown, n, true, tmp);
+    unsigned long long *dof = row0;  // the raw rows' places are done with
+    if (int r = exclusive_sum(tmp, dof)) return r;
+    uint64_t entries = 0;
+    if (int r = read_word(dof + n, entries)) return r;
+    const uint64_t nunits = (entries + kUnit - 1) / kUnit;
+    // the lists take the raw rows' memory: two words an entry, at most one
+    // entry per undirected edge of a graph that holds both directions
+    if (!fits(raw, std::max<uint64_t>(entries, 1) * 8) ||
+        !fits(units, std::max<uint64_t>(nunits, 1) * 4) || !fits(grabs, kTakers * 128))
+      return MK_OK;
+    if (entries) {
+      unsigned long long *down = raw.as<unsigned long long>();
+      k_tc_down<<<grid, kBlock, 0, stream>>>(len, off, uplist.as<uint32_t>(), slot.as<uint32_t>(),
+                                             dof, n, down);
+      k_tc_units<<<tgrid, kBlock, 0, stream>>>(dof, n, units.as<uint32_t>());
+      uint64_t stride = 1;
+      if (nunits > 2) {
+        stride = uint64_t(double(nunits) * 0.6180339887) | 1u;
+        while (std::gcd(stride, nunits) != 1) stride += 2;
+        stride %= nunits;
+      }
+      fill_u64(grabs.as<uint64_t>(), 0ull, kTakers * 16, stream);
+      ProfScope prof2(stream, "k_tc_intersect", 0.0);
+      const unsigned wgrid = blocks_for_waves(
+          std::min<uint64_t>(nunits, uint64_t(device_cus(g->device)) * 32));
+      k_tc_wedges<<<wgrid, kBlock, 0, stream>>>(len, off, uplist.as<uint32_t>(), dof, down,
+                                                units.as<uint32_t>(), n, entries, nunits, stride,
+                                                grabs.as<unsigned long long>(), slots);
+    }
+    MK_HIP(hipGetLastError());
+    *done = true;
+    return MK_OK;
+  }
+
   int run_static(float *ms) {
     if (int r = start()) return r;
+    bool done = false;
+    if (int r = queue_wedges(&done)) return r;
+    if (done) {
+      uint64_t t = 0;
+      if (int r = finish(t, ms)) return r;
+      if (profiling_on()) prof_add_bytes("k_tc_lists", 256.0 * double(last_slabs));
+      count = t;
+      return MK_OK;
+    }
+    return run_static_lists(ms);
+  }
+
+  // Static count without the sorted rows: 4 bytes of scratch an undirected
+  // edge.
+  int run_static_lists(float *ms) {
+    fill_u64(reinterpret_cast<uint64_t *>(slots), 0ull, kTcSlots + 2, stream);
     const size_t n = g->n;
     if (int r = kup.ensure((n + 1) * 8)) return r;
     if (int r = koff.ensure((n + 1) * 8)) return r;
