@@ -46,49 +46,12 @@ MK_DEV bool rank_lt(uint32_t da, uint32_t a, uint32_t db, uint32_t b) {
   return da < db || (da == db && a < b);
 }
 
-// Lanes with `act` hold key c: returns whether c is a live key of vertex y.
-// Lanes targeting the same bucket of y share one walk of its chain.
-// Wave-collective.
-template <bool MAP>
-MK_DEV bool probe_member(const GraphView &G, uint32_t y, bool act, uint32_t c, uint32_t &slabs) {
-  const uint32_t lane = lane_id();
-  const uint32_t off = G.bucket_off[y], nb = G.bucket_off[y + 1] - off;
-  const uint64_t km = key_mask<MAP>();
-  const uint32_t bk = act ? off + bucket_in(c, nb) : 0u;
-  bool hit = false;
-  uint64_t pending = ballot(act);
-  while (pending) {
-    const uint32_t bb = read_lane(bk, ffs64(pending));
-    const bool mine = act && bk == bb;
-    pending &= ~ballot(mine);
-    const uint64_t mm = ballot(mine);
-    const uint32_t *slab = G.heads + size_t(bb) * kSlabWords;
-    for (;;) {
-      const uint32_t x = slab[lane];
-      ++slabs;
-      uint64_t live = ballot(x < kTomb) & km;
-      if (__popcll(mm) < __popcll(live)) {
-        // few candidates: broadcast each and compare with the whole slab
-        uint64_t t = mm;
-        while (t) {
-          const uint32_t j = ffs64(t);
-          t &= t - 1;
-          const uint32_t cj = read_lane(c, j);
-          if (ballot(x == cj) & live) hit |= lane == j;
-        }
-      } else {
-        while (live) {
-          const uint32_t k = ffs64(live);
-          live &= live - 1;
-          hit |= mine && c == read_lane(x, k);
-        }
-      }
-      const uint32_t nx = read_lane(x, kNextLane);
-      if (nx == kEmpty) break;
-      slab = slab_ptr(G.pool, nx);
-    }
-  }
-  return hit;
+// Orders the wave's LDS accesses before and after it (the LDS unit takes a
+// wave's accesses in order: no instruction, the compiler only).
+MK_DEV void lds_settle() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 MK_DEV uint64_t edge_key(uint32_t a, uint32_t b) {
@@ -296,14 +259,6 @@ constexpr uint32_t kTakers = 16;         // unit counters
 constexpr uint32_t kSortRow = 1024;     // row elements staged in LDS at a time
 constexpr uint32_t kTail = 8;           // lanes per tail
 constexpr uint32_t kRounds = 4;         // elements a lane takes at a time
-
-// Orders the wave's LDS accesses before and after it (the LDS unit takes a
-// wave's accesses in order: no instruction, the compiler only).
-MK_DEV void lds_settle() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 __global__ void k_tc_iota(uint32_t *p, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -650,13 +605,20 @@ __global__ void __launch_bounds__(kBlock)
   if (lane == 0) add_count(slots, count);
 }
 
+// The end of a changed edge that is enumerated (x, fewer live neighbours) and
+// the one that is tested (y).
+MK_DEV uint2 tc_ends(const GraphView &G, uint2 uv) {
+  return G.vdeg[uv.x] > G.vdeg[uv.y] ? make_uint2(uv.y, uv.x) : uv;
+}
+
 // Canonical changed edges of a batch: entries with status == APPLIED (or all
 // non-loop entries when status is NULL) enter the set; the first entry of
-// each undirected edge appends it to `owned`.
+// each undirected edge appends it to `owned` and adds the buckets of its
+// enumerated end to *n_items.
 __global__ void __launch_bounds__(kBlock)
-    k_tc_collect(const uint32_t *src, const uint32_t *dst, const uint8_t *status, uint32_t n,
+    k_tc_collect(GraphView G, const uint32_t *src, const uint32_t *dst, const uint8_t *status, uint32_t n,
                  uint32_t nv, unsigned long long *tab, uint32_t mask, uint2 *owned,
-                 uint32_t *n_owned) {
+                 uint32_t *n_owned, unsigned long long *n_items) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   bool mine = false;
   uint32_t u = 0, v = 0;
@@ -673,55 +635,129 @@ __global__ void __launch_bounds__(kBlock)
     if (lane_id() == leader) base = atomicAdd(n_owned, uint32_t(__popcll(m)));
     base = read_lane(base, leader);
     if (mine) owned[base + lanes_below(m)] = make_uint2(min(u, v), max(u, v));
+    uint32_t nb = 0;
+    if (mine) {
+      const uint32_t x = tc_ends(G, make_uint2(min(u, v), max(u, v))).x;
+      nb = G.bucket_off[x + 1] - G.bucket_off[x];
+    }
+    const uint64_t sum = wave_sum_u64(nb);
+    if (lane_id() == leader) atomicAdd(n_items, (unsigned long long)sum);
   }
+}
+
+// Work items of the changed edges: (edge, bucket of its enumerated end), the
+// edge's items side by side; one claim on *next per wave.
+__global__ void __launch_bounds__(kBlock)
+    k_tc_items(GraphView G, const uint2 *owned, uint32_t n_owned, uint2 *items,
+               unsigned long long *next) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t lane = lane_id();
+  uint32_t nb = 0;
+  if (i < n_owned) {
+    const uint32_t x = tc_ends(G, owned[i]).x;
+    nb = G.bucket_off[x + 1] - G.bucket_off[x];
+  }
+  uint64_t incl = nb;
+#pragma unroll
+  for (uint32_t o = 1; o < 64; o <<= 1) {
+    const uint64_t y = (uint64_t(uint32_t(__shfl_up(int(incl >> 32), o, 64))) << 32) |
+                       uint32_t(__shfl_up(int(uint32_t(incl)), o, 64));
+    if (lane >= o) incl += y;
+  }
+  unsigned long long base = 0;
+  if (lane == 63) base = atomicAdd(next, (unsigned long long)incl);
+  base = (uint64_t(read_lane(uint32_t(base >> 32), 63)) << 32) | read_lane(uint32_t(base), 63);
+  for (uint32_t j = 0; j < nb; ++j) items[base + incl - nb + j] = make_uint2(i, j);
 }
 
 // Weight of a triangle with j changed edges: 6 / j.
 MK_DEV uint32_t six_over(uint32_t j) { return j == 1 ? 6u : (j == 2 ? 3u : 2u); }
 
-// Triangles through each inserted edge {u, v} (graph already updated):
-// w over adj[x] of the lower-degree end x, tested in adj[y].
+// Test the keys c of the lanes with `act` against vertex y's adjacency: the
+// keys are packed into LDS and each 8-lane group tests two at a time, so
+// that sixteen of y's slabs are in flight per wave (a wave-wide walk had one:
+// a key and its slab after the other).  Returns whether this lane's key is
+// there.  Wave-collective.
+template <bool MAP>
+MK_DEV bool tc_test_keys(const GraphView &G, uint32_t y, bool act, uint32_t c, uint32_t *lds,
+                         uint32_t &slabs) {
+  const uint32_t gl = group_lane(), grp = lane_id() / kGroupLanes;
+  const uint64_t m = ballot(act);
+  const uint32_t n = uint32_t(__popcll(m));
+  lds_settle();
+  if (act) lds[lanes_below(m)] = c;
+  lds_settle();
+  const uint32_t off = G.bucket_off[y], nb = G.bucket_off[y + 1] - off;
+  for (uint32_t k0 = 0; k0 < n; k0 += 2 * kGroupsPerWave) {
+    uint32_t key[2], v[2][kWordsPerLane];
+#pragma unroll
+    for (uint32_t q = 0; q < 2; ++q) {
+      const uint32_t k = k0 + q * kGroupsPerWave + grp;
+      key[q] = k < n ? lds[k] : kEmpty;
+      if (key[q] != kEmpty)
+        load_words(G.heads + size_t(off + bucket_in(key[q], nb)) * kSlabWords + kWordsPerLane * gl,
+                   v[q]);
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < 2; ++q) {
+      if (key[q] == kEmpty) continue;
+      bool found = false;
+      for (;;) {
+        if (gl == 0) ++slabs;
+        bool hit = false;
+#pragma unroll
+        for (uint32_t j = 0; j < kWordsPerLane; ++j)
+          hit |= key_word<MAP>(kWordsPerLane * gl + j) && v[q][j] == key[q];
+        found = group_bits(ballot(hit)) != 0u;
+        const uint32_t nx = group_read(v[q][kWordsPerLane - 1], kGroupLanes - 1);
+        if (found || nx == kEmpty) break;
+        load_words(slab_ptr(G.pool, nx) + kWordsPerLane * gl, v[q]);
+      }
+      if (gl == 0) lds[k0 + q * kGroupsPerWave + grp] = found ? 1u : 0u;
+    }
+  }
+  lds_settle();
+  return act && lds[lanes_below(m)] != 0u;
+}
+
+// Triangles through each inserted edge {u, v} (graph already updated): w
+// over adj[x] of the lower-degree end x, tested in adj[y]; a wave per item
+// (edge, bucket of x), so that a hub's buckets are spread over the device.
+// Bound by the latency of y's slabs.  RMAT-18, 50k edges of the same
+// distribution: 0.38 ms; 1.64 ms with a wave per edge (the hub edges'
+// waves ran last, alone) that tested a key after the other.
 template <bool MAP>
 __global__ void __launch_bounds__(kBlock)
-    k_tc_inserted(GraphView G, const uint2 *owned, uint32_t n_owned,
+    k_tc_inserted(GraphView G, const uint2 *owned, const uint2 *items, uint64_t n_items,
                   const unsigned long long *tab, uint32_t mask, unsigned long long *slots,
                   unsigned long long *slab_count) {
+  __shared__ uint32_t keys[kBlock / 64][64];
+  uint32_t *lds = keys[threadIdx.x >> 6];
   const uint32_t lane = lane_id();
-  const uint32_t gw = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const uint32_t W = (gridDim.x * blockDim.x) >> 6;
+  const uint64_t gw = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
+  const uint64_t W = (uint64_t(gridDim.x) * blockDim.x) >> 6;
   const bool key_lane = (key_mask<MAP>() >> lane) & 1ull;
   uint64_t count = 0;
   uint32_t slabs = 0;
-  for (uint32_t e = gw; e < n_owned; e += W) {
-    const uint2 uv = owned[e];
-    uint32_t x = uv.x, y = uv.y;
-    if (G.vdeg[x] > G.vdeg[y]) {
-      const uint32_t t = x;
-      x = y;
-      y = t;
-    }
-    for (uint32_t bk = G.bucket_off[x]; bk < G.bucket_off[x + 1]; ++bk) {
-      const uint32_t *slab = G.heads + size_t(bk) * kSlabWords;
-      for (;;) {
-        const uint32_t w = slab[lane];
-        ++slabs;
-        const bool act = key_lane && w < kTomb && w != y;
-        if (ballot(act)) {
-          const bool hit = probe_member<MAP>(G, y, act, w, slabs);
-          uint32_t add = 0;
-          if (hit) {
-            const uint32_t j = 1u + (set_contains(tab, mask, edge_key(x, w)) ? 1u : 0u) +
-                               (set_contains(tab, mask, edge_key(y, w)) ? 1u : 0u);
-            add = six_over(j);
-          }
-          count += wave_sum_u32(add);
-        }
-        const uint32_t nx = read_lane(w, kNextLane);
-        if (nx == kEmpty) break;
-        slab = slab_ptr(G.pool, nx);
-      }
+  for (uint64_t t = gw; t < n_items; t += W) {
+    const uint2 it = items[t];
+    const uint2 xy = tc_ends(G, owned[it.x]);
+    const uint32_t x = xy.x, y = xy.y;
+    const uint32_t *slab = G.heads + size_t(G.bucket_off[x] + it.y) * kSlabWords;
+    for (;;) {
+      const uint32_t w = slab[lane];
+      if (lane == 0) ++slabs;
+      const bool act = key_lane && w < kTomb && w != y;
+      if (tc_test_keys<MAP>(G, y, act, w, lds, slabs))
+        count += six_over(1u + (set_contains(tab, mask, edge_key(x, w)) ? 1u : 0u) +
+                          (set_contains(tab, mask, edge_key(y, w)) ? 1u : 0u));
+      const uint32_t nx = read_lane(w, kNextLane);
+      if (nx == kEmpty) break;
+      slab = slab_ptr(G.pool, nx);
     }
   }
+  count = wave_sum_u64(count);
+  slabs = wave_sum_u32(slabs);
   if (lane == 0) {
     add_count(slots, count);
     if (slabs) atomicAdd(slab_count, (unsigned long long)slabs);
@@ -747,69 +783,54 @@ __global__ void k_tc_dfill(const uint2 *owned, uint32_t n_owned, const uint32_t 
 
 // Triangles of the graph before the delete through each deleted edge
 // {u, v}: w over (current adj[x]) + (deleted neighbours of x), tested
-// against (current adj[y]) + (deleted neighbours of y, via the set).
+// against (current adj[y]) + (deleted neighbours of y, via the set).  Items
+// as in k_tc_inserted; x's deleted neighbours are shared out over its items
+// 64 at a time.  RMAT-18, 50k edges: 1.62 -> 0.56 ms.
 template <bool MAP>
 __global__ void __launch_bounds__(kBlock)
-    k_tc_deleted(GraphView G, const uint2 *owned, uint32_t n_owned,
+    k_tc_deleted(GraphView G, const uint2 *owned, const uint2 *items, uint64_t n_items,
                  const unsigned long long *tab, uint32_t mask, const uint32_t *doff,
                  const uint32_t *dlist, unsigned long long *slots, unsigned long long *slab_count) {
+  __shared__ uint32_t keys[kBlock / 64][64];
+  uint32_t *lds = keys[threadIdx.x >> 6];
   const uint32_t lane = lane_id();
-  const uint32_t gw = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const uint32_t W = (gridDim.x * blockDim.x) >> 6;
+  const uint64_t gw = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
+  const uint64_t W = (uint64_t(gridDim.x) * blockDim.x) >> 6;
   const bool key_lane = (key_mask<MAP>() >> lane) & 1ull;
   uint64_t count = 0;
   uint32_t slabs = 0;
-  for (uint32_t e = gw; e < n_owned; e += W) {
-    const uint2 uv = owned[e];
-    uint32_t x = uv.x, y = uv.y;
-    const uint32_t cx = G.vdeg[x] + (doff[x + 1] - doff[x]);
-    const uint32_t cy = G.vdeg[y] + (doff[y + 1] - doff[y]);
-    if (cx > cy) {
-      const uint32_t t = x;
-      x = y;
-      y = t;
-    }
+  for (uint64_t t = gw; t < n_items; t += W) {
+    const uint2 it = items[t];
+    const uint2 xy = tc_ends(G, owned[it.x]);
+    const uint32_t x = xy.x, y = xy.y;
+    // the changed edges of triangle {x, y, w}: {x, y}, {x, w} in part (b),
+    // and {y, w} if it was deleted (then it is not in adj[y] now)
+    auto tally = [&](bool act, uint32_t w, uint32_t changed) {
+      const bool gone = act && set_contains(tab, mask, edge_key(y, w));
+      const bool found = tc_test_keys<MAP>(G, y, act, w, lds, slabs);
+      if (found || gone) count += six_over(changed + (gone ? 1u : 0u));
+    };
     // (a) w in the current adjacency of x: {x, w} is not deleted
-    for (uint32_t bk = G.bucket_off[x]; bk < G.bucket_off[x + 1]; ++bk) {
-      const uint32_t *slab = G.heads + size_t(bk) * kSlabWords;
-      for (;;) {
-        const uint32_t w = slab[lane];
-        ++slabs;
-        const bool act = key_lane && w < kTomb && w != y;
-        if (ballot(act)) {
-          const bool in_now = probe_member<MAP>(G, y, act, w, slabs);
-          uint32_t add = 0;
-          if (act) {
-            const bool yw_del = set_contains(tab, mask, edge_key(y, w));
-            if (in_now || yw_del) add = six_over(1u + (yw_del ? 1u : 0u));
-          }
-          count += wave_sum_u32(add);
-        }
-        const uint32_t nx = read_lane(w, kNextLane);
-        if (nx == kEmpty) break;
-        slab = slab_ptr(G.pool, nx);
-      }
+    const uint32_t b0 = G.bucket_off[x], nb = G.bucket_off[x + 1] - b0;
+    const uint32_t *slab = G.heads + size_t(b0 + it.y) * kSlabWords;
+    for (;;) {
+      const uint32_t w = slab[lane];
+      if (lane == 0) ++slabs;
+      tally(key_lane && w < kTomb && w != y, w, 1u);
+      const uint32_t nx = read_lane(w, kNextLane);
+      if (nx == kEmpty) break;
+      slab = slab_ptr(G.pool, nx);
     }
     // (b) w a deleted neighbour of x: {x, w} is deleted
     const uint32_t d0 = doff[x], d1 = doff[x + 1];
-    for (uint32_t j0 = d0; j0 < d1; j0 += 64) {
-      const uint32_t j = j0 + lane;
-      uint32_t w = 0;
-      bool act = false;
-      if (j < d1) {
-        w = dlist[j];
-        act = w != y;
-      }
-      if (ballot(act) == 0) continue;
-      const bool in_now = probe_member<MAP>(G, y, act, w, slabs);
-      uint32_t add = 0;
-      if (act) {
-        const bool yw_del = set_contains(tab, mask, edge_key(y, w));
-        if (in_now || yw_del) add = six_over(2u + (yw_del ? 1u : 0u));
-      }
-      count += wave_sum_u32(add);
+    for (uint64_t j0 = d0 + uint64_t(it.y) * 64; j0 < d1; j0 += uint64_t(nb) * 64) {
+      const uint64_t j = j0 + lane;
+      const uint32_t w = j < d1 ? dlist[j] : y;
+      tally(w != y, w, 2u);
     }
   }
+  count = wave_sum_u64(count);
+  slabs = wave_sum_u32(slabs);
   if (lane == 0) {
     add_count(slots, count);
     if (slab_count && slabs) atomicAdd(slab_count, (unsigned long long)slabs);
@@ -822,8 +843,9 @@ struct TC {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // kTcSlots counts, then the slab counter and the streamed-elements counter
   unsigned long long *slots = nullptr;
-  uint32_t *n_owned = nullptr;
+  uint32_t *n_owned = nullptr;  // [0] changed edges, [2..3] their items, [4..5] items written
   DevBuf tab, owned, ddeg, doff, cursor, dlist, scan_tmp, kup, koff, uplist, grabs;
+  DevBuf items;
   DevBuf ranks, rows, raw, slot, units;  // static count over sorted rows
   HostBuf host;
   unsigned long long count = 0;
@@ -838,7 +860,7 @@ struct TC {
     MK_HIP(hipEventCreate(&ev0));
     MK_HIP(hipEventCreate(&ev1));
     MK_HIP(hipMalloc(&slots, (kTcSlots + 2) * 8));
-    MK_HIP(hipMalloc(&n_owned, 4));
+    MK_HIP(hipMalloc(&n_owned, 32));
     if (int r = host.ensure((kTcSlots + 3) * 8)) return r;
     max_waves = grid_waves(g->device);
     return MK_OK;
@@ -851,7 +873,7 @@ struct TC {
     (void)hipFree(n_owned);
     for (DevBuf *b :
          {&tab, &owned, &ddeg, &doff, &cursor, &dlist, &scan_tmp, &kup, &koff, &uplist, &grabs,
-          &ranks, &rows, &raw, &slot, &units})
+          &items, &ranks, &rows, &raw, &slot, &units})
       b->release();
     host.release();
     if (ev0) (void)hipEventDestroy(ev0);
@@ -1066,23 +1088,31 @@ struct TC {
 
   // Changed undirected edges of the batch into the set; returns their count.
   int collect(const uint32_t *src, const uint32_t *dst, uint32_t n, int op, uint32_t &mask,
-              uint32_t &m) {
+              uint32_t &m, uint64_t &nitems) {
     uint32_t cap = 1024;
     while (cap < 2ull * n) cap <<= 1;
     mask = cap - 1;
     if (int r = tab.ensure(size_t(cap) * 8)) return r;
     if (int r = owned.ensure(size_t(std::max(n, 1u)) * 8)) return r;
     fill_u64(tab.as<uint64_t>(), ~0ull, cap, stream);
-    fill_u32(n_owned, 0u, 1, stream);
+    fill_u32(n_owned, 0u, 8, stream);
+    unsigned long long *n_items = reinterpret_cast<unsigned long long *>(n_owned + 2);
     const bool same = g->last_op == op && g->last_src == src && g->last_dst == dst &&
                       g->status_n == n;
     const uint8_t *st = same ? g->status.as<uint8_t>() : nullptr;
     k_tc_collect<<<blocks_for_threads(n), kBlock, 0, stream>>>(
-        src, dst, st, n, g->n, tab.as<unsigned long long>(), mask, owned.as<uint2>(), n_owned);
+        g->view(), src, dst, st, n, g->n, tab.as<unsigned long long>(), mask, owned.as<uint2>(),
+        n_owned, n_items);
     MK_HIP(hipGetLastError());
-    MK_HIP(hipMemcpyAsync(host.ptr, n_owned, 4, hipMemcpyDeviceToHost, stream));
+    MK_HIP(hipMemcpyAsync(host.ptr, n_owned, 16, hipMemcpyDeviceToHost, stream));
     MK_HIP(hipStreamSynchronize(stream));
-    m = *host.as<uint32_t>();
+    m = host.as<uint32_t>()[0];
+    nitems = host.as<uint64_t>()[1];
+    if (m) {
+      if (int r = items.ensure(nitems * 8)) return r;
+      k_tc_items<<<blocks_for_threads(m), kBlock, 0, stream>>>(
+          g->view(), owned.as<uint2>(), m, items.as<uint2>(), n_items + 1);
+    }
     return MK_OK;
   }
 
@@ -1092,18 +1122,15 @@ struct TC {
     uint64_t t = 0;
     if (n) {
       uint32_t mask = 0, m = 0;
-      if (int r = collect(src, dst, n, 1, mask, m)) return r;
+      uint64_t ni = 0;
+      if (int r = collect(src, dst, n, 1, mask, m, ni)) return r;
       if (m) {
-        const unsigned grid = blocks_for_waves(std::min<uint64_t>(m, uint64_t(max_waves) * 2));
+        const unsigned grid = blocks_for_waves(std::min<uint64_t>(ni, uint64_t(max_waves) * 2));
         ProfScope prof(stream, "k_tc_inserted", 0.0);
-        if (g->weighted)
-          k_tc_inserted<true><<<grid, kBlock, 0, stream>>>(g->view(), owned.as<uint2>(), m,
-                                                          tab.as<unsigned long long>(), mask,
-                                                          slots, slots + kTcSlots);
-        else
-          k_tc_inserted<false><<<grid, kBlock, 0, stream>>>(g->view(), owned.as<uint2>(), m,
-                                                           tab.as<unsigned long long>(), mask,
-                                                           slots, slots + kTcSlots);
+        auto k = g->weighted ? k_tc_inserted<true> : k_tc_inserted<false>;
+        k<<<grid, kBlock, 0, stream>>>(g->view(), owned.as<uint2>(), items.as<uint2>(), ni,
+                                       tab.as<unsigned long long>(), mask, slots,
+                                       slots + kTcSlots);
       }
     }
     if (int r = finish(t, ms)) return r;
@@ -1118,7 +1145,8 @@ struct TC {
     uint64_t t = 0;
     if (n) {
       uint32_t mask = 0, m = 0;
-      if (int r = collect(src, dst, n, 2, mask, m)) return r;
+      uint64_t ni = 0;
+      if (int r = collect(src, dst, n, 2, mask, m, ni)) return r;
       if (m) {
         // CSR of the deleted edges (both directions)
         const size_t nv = g->n;
@@ -1139,16 +1167,12 @@ struct TC {
         k_tc_dfill<<<blocks_for_threads(m), kBlock, 0, stream>>>(
             owned.as<uint2>(), m, doff.as<uint32_t>(), cursor.as<uint32_t>(),
             dlist.as<uint32_t>());
-        const unsigned grid = blocks_for_waves(std::min<uint64_t>(m, uint64_t(max_waves) * 2));
+        const unsigned grid = blocks_for_waves(std::min<uint64_t>(ni, uint64_t(max_waves) * 2));
         ProfScope prof(stream, "k_tc_deleted", 0.0);
-        if (g->weighted)
-          k_tc_deleted<true><<<grid, kBlock, 0, stream>>>(
-              g->view(), owned.as<uint2>(), m, tab.as<unsigned long long>(), mask,
-              doff.as<uint32_t>(), dlist.as<uint32_t>(), slots, slots + kTcSlots);
-        else
-          k_tc_deleted<false><<<grid, kBlock, 0, stream>>>(
-              g->view(), owned.as<uint2>(), m, tab.as<unsigned long long>(), mask,
-              doff.as<uint32_t>(), dlist.as<uint32_t>(), slots, slots + kTcSlots);
+        auto k = g->weighted ? k_tc_deleted<true> : k_tc_deleted<false>;
+        k<<<grid, kBlock, 0, stream>>>(g->view(), owned.as<uint2>(), items.as<uint2>(), ni,
+                                       tab.as<unsigned long long>(), mask, doff.as<uint32_t>(),
+                                       dlist.as<uint32_t>(), slots, slots + kTcSlots);
       }
     }
     if (int r = finish(t, ms)) return r;

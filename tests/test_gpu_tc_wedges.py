@@ -62,3 +62,37 @@ def test_scratch_bound_selects_plain_lists(gpu):
             assert count(n, s, d) == want
     finally:
         _lib.call("mk_tune_set", b"tc_scratch_mb", old.value)
+
+
+@pytest.mark.parametrize("weighted,hints", [(False, True), (True, True), (False, False)])
+def test_batches_through_hubs(gpu, weighted, hints):
+    # two hubs of several buckets (one bucket and long chains without hints)
+    # joined, split and joined again within a batch: hub-hub edges, all of a
+    # vertex's edges deleted, the batch's own edges closing triangles
+    n, s, d, _ = gen.rmat(12, 8, seed=3, undirected=True)
+    hub = np.arange(2, n - 5, dtype=np.uint32)  # the last vertices stay isolated
+    a = np.r_[np.full(len(hub), 0), np.full(len(hub), 1), [0]].astype(np.uint32)
+    b = np.r_[hub, hub, [1]].astype(np.uint32)
+    more = np.unique(np.r_[gen.keys_of(a, b), gen.keys_of(b, a)])
+    base = np.setdiff1d(gen.keys_of(s, d), more)
+    S, D = gen.split_keys(base)
+    allS, _ = gen.split_keys(np.union1d(base, more))
+    one = np.ones(len(base) + len(more), np.uint32) if weighted else None
+    pool = mk.SlabPool(1 << 27)
+    g = mk.DynamicGraph(n, pool, 0.7, gen.degree_hints(n, allS) if hints else None,
+                        weighted=weighted)
+    g.InsertEdges(S, D, one[:len(S)] if weighted else None)
+    tc = mk.TC(g)
+    tc.Static()
+    small = oracle.tc(oracle.csr(n, S, D))
+    full = oracle.tc(oracle.csr(n, *gen.split_keys(np.union1d(base, more))))
+    assert tc.GetCount() == small
+    ms, md = (mk.device_u32(x) for x in gen.split_keys(more))
+    mw = mk.device_u32(one[:len(more)]) if weighted else None
+    for _ in range(2):
+        g.InsertEdges(ms, md, mw)
+        tc.Incremental(ms, md)
+        assert tc.GetCount() == full
+        g.DeleteEdges(ms, md)
+        tc.Decremental(ms, md)
+        assert tc.GetCount() == small
