@@ -9,8 +9,12 @@
 // variants, :24-86): a halving store only replaces a parent by one of its
 // ancestors, which keeps parent[x] <= x, so concurrent halving is safe.
 //
-// Edges are taken as undirected (weak components).  Static = union over
-// every edge in the slabs, then a compress pass (label = root).  Incremental
+// Edges are taken as undirected (weak components).  Static = union over one
+// or two edges of every vertex, a compress pass (label = root), union over
+// the edges in the slabs whose ends' labels still differ (the sampling of
+// Sutton, Ben-Nun and Barak, "Optimizing parallel graph connectivity
+// computation via subgraph sampling", IPDPS 2018; every edge is looked at,
+// since a graph may hold an edge in one direction only), compress again.  Incremental
 // = union over the inserted batch, then compress.  Decremental recomputes
 // (union-find cannot split components).
 #include <hip/hip_runtime.h>
@@ -68,55 +72,103 @@ MK_DEV void uf_union(uint32_t *parent, uint32_t a, uint32_t b) {
   }
 }
 
+// Sampling steps before the edge pass.  Whole static passes, against finds
+// for both ends of every edge: RMAT-21 1.79 -> 0.67 ms, RMAT-18 0.64 -> 0.10,
+// ER 1M x 16M 0.76 -> 0.63, ER 1M x 1M 0.98 -> 0.33, a path of 1M vertices
+// 0.90 -> 0.14, a grid of 1M 0.69 -> 0.15.
+constexpr uint32_t kSampleSteps = 3;
+constexpr uint32_t kHookBlock = 1024;
+
 __global__ void k_cc_init(uint32_t *parent, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) parent[i] = i;
 }
 
-// Union over every edge: waves stream over buckets 64 at a time; each slab
-// is loaded once and its keys united with the bucket's owner lane-parallel.
+// Keys of vertex u in words `word`, +1, +16 and +17 of its first slab (a map:
+// two of them): with word 0 the first that inserts fill.  kEmpty: none.
+template <bool MAP> MK_DEV void first_keys(const GraphView &G, uint32_t u, uint32_t word,
+                                           uint32_t (&k)[4]) {
+  const uint32_t *slab = G.heads + size_t(G.bucket_off[u]) * kSlabWords + word;
+  const uint2 a = *reinterpret_cast<const uint2 *>(slab);
+  const uint2 b = *reinterpret_cast<const uint2 *>(slab + 16);
+  k[0] = a.x < kTomb ? a.x : kEmpty;
+  k[1] = !MAP && a.y < kTomb ? a.y : kEmpty;
+  k[2] = b.x < kTomb ? b.x : kEmpty;
+  k[3] = !MAP && b.y < kTomb ? b.y : kEmpty;
+}
+
+// Sampling step 0: every vertex hangs under the smallest of itself and its
+// first keys (a forest: parents are smaller); parents within the block's
+// vertices are followed in LDS right away, so that neighbours in id order
+// (paths, grids) make no long chains for the compress pass.
+template <bool MAP>
+__global__ void __launch_bounds__(kHookBlock) k_cc_hook(GraphView G, uint32_t *parent) {
+  __shared__ uint32_t lp[kHookBlock];
+  const uint32_t t = threadIdx.x, base = blockIdx.x * kHookBlock, u = base + t;
+  uint32_t p = u;
+  if (u < G.n && G.vdeg[u] != 0) {
+    uint32_t k[4];
+    first_keys<MAP>(G, u, 0, k);
+    p = min(min(min(k[0], k[1]), min(k[2], k[3])), u);
+  }
+#pragma unroll 1
+  for (uint32_t len = 1; len < kHookBlock; len <<= 1) {  // pointer doubling
+    lp[t] = p;
+    __syncthreads();
+    if (p >= base) p = lp[p - base];
+    __syncthreads();
+  }
+  if (u < G.n) parent[u] = p;
+}
+
+// Sampling steps 1, 2, ..., paths shortened in between: the vertex's label
+// (a root, mostly) takes the smallest label among its keys in words `word`, if that
+// is smaller.  Of several offers to one root the smallest stays; the edges
+// of the others join in a later step or in k_cc_edges.  No step waits or
+// retries: finds and CAS loops from every vertex at once made chains that
+// took 0.3 ms on RMAT-21 and 8 ms on a path of 1M vertices.
+template <bool MAP>
+__global__ void k_cc_sample(GraphView G, uint32_t *parent, uint32_t word) {
+  const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= G.n || G.vdeg[u] == 0) return;
+  uint32_t k[4];
+  first_keys<MAP>(G, u, word, k);
+  const uint32_t pu = parent[u];
+  uint32_t lo = pu;
+#pragma unroll
+  for (uint32_t q = 0; q < 4; ++q)
+    if (k[q] != kEmpty) lo = min(lo, parent[k[q]]);
+  if (lo < pu && coherent_load(parent + pu) > lo) atomicMin(parent + pu, lo);
+}
+
+// Union over the edges whose ends have different labels: an 8-lane group per
+// bucket, a slab's neighbour labels gathered together (eight slabs in flight
+// per wave).  Labels were shortened to roots before, so almost every edge
+// ends at that gather; equal labels always mean one component, and where
+// they differ the union looks for the roots.  Bound by the gathers (4 bytes from an
+// array of 4 bytes a vertex): RMAT-21, 62M stored edges, 0.43 ms.
 template <bool MAP>
 __global__ void __launch_bounds__(kBlock) k_cc_edges(GraphView G, uint32_t *parent) {
-  const uint32_t lane = lane_id();
-  const uint32_t gw = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const uint32_t W = (gridDim.x * blockDim.x) >> 6;
-  const bool key_lane = (key_mask<MAP>() >> lane) & 1ull;
-  for (uint64_t b0 = uint64_t(gw) * 64; b0 < G.total_buckets; b0 += uint64_t(W) * 64) {
-    const uint64_t b = b0 + lane;
-    bool act = b < G.total_buckets;
-    uint32_t u = 0;
-    if (act) {
-      u = G.bucket_owner[b];
-      act = G.vdeg[u] != 0;
-    }
-    uint64_t m = ballot(act);
-    while (m) {
-      uint32_t js[4];
-      uint32_t c = 0;
+  const uint32_t gl = group_lane();
+  const uint64_t g0 = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kGroupLanes;
+  const uint64_t NG = uint64_t(gridDim.x) * blockDim.x / kGroupLanes;
+  for (uint64_t b = g0; b < G.total_buckets; b += NG) {
+    const uint32_t u = G.bucket_owner[b];
+    if (G.vdeg[u] == 0) continue;
+    const uint32_t pu = parent[u];
+    const uint32_t *slab = G.heads + b * kSlabWords;
+    for (;;) {
+      uint32_t x[kWordsPerLane], px[kWordsPerLane];
+      load_words(slab + kWordsPerLane * gl, x);
 #pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) {
-        js[k] = m ? ffs64(m) : 0u;
-        if (m) {
-          m &= m - 1;
-          c = k + 1;
-        }
-      }
-      uint32_t x[4];
+      for (uint32_t k = 0; k < kWordsPerLane; ++k)
+        px[k] = key_word<MAP>(kWordsPerLane * gl + k) && x[k] < kTomb ? parent[x[k]] : pu;
 #pragma unroll
-      for (uint32_t k = 0; k < 4; ++k)
-        x[k] = k < c ? G.heads[(b0 + js[k]) * kSlabWords + lane] : kEmpty;
-#pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) {
-        if (k >= c) continue;
-        const uint32_t uj = read_lane(u, js[k]);
-        uint32_t v = x[k];
-        for (;;) {
-          if (key_lane && v < kTomb) uf_union(parent, uj, v);
-          const uint32_t nx = read_lane(v, kNextLane);
-          if (nx == kEmpty) break;
-          v = slab_ptr(G.pool, nx)[lane];
-        }
-      }
+      for (uint32_t k = 0; k < kWordsPerLane; ++k)
+        if (px[k] != pu) uf_union(parent, u, x[k]);
+      const uint32_t nx = group_read(x[kWordsPerLane - 1], kGroupLanes - 1);
+      if (nx == kEmpty) break;
+      slab = slab_ptr(G.pool, nx);
     }
   }
 }
@@ -137,6 +189,15 @@ __global__ void k_cc_compress(uint32_t *parent, uint32_t n) {
   uint32_t r = parent[i];
   while (parent[r] != r) r = parent[r];
   parent[i] = r;
+}
+
+// The same between sampling steps, halving paths on the way, so that the
+// threads of a long chain shorten it together.  A halving store may land
+// after another thread's and leave an ancestor that is not the root: no
+// harm to the steps that follow, but labels end with k_cc_compress.
+__global__ void k_cc_shorten(uint32_t *parent, uint32_t n) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) parent[i] = uf_find(parent, i);
 }
 
 struct CC {
@@ -188,15 +249,28 @@ struct CC {
   int run_static(float *ms) {
     MK_HIP(hipSetDevice(g->device));
     MK_HIP(hipEventRecord(ev0, stream));
-    k_cc_init<<<blocks_for_threads(g->n), kBlock, 0, stream>>>(parent, g->n);
     const unsigned grid = blocks_for_waves(std::min<uint64_t>(
-        (uint64_t(g->total_buckets) + 63) / 64, uint64_t(device_cus(g->device)) * 16));
+        (uint64_t(g->total_buckets) + 7) / 8, uint64_t(device_cus(g->device)) * 32));
     {
-      // per bucket: owner + degree (8 B) and its slabs; per edge two root
-      // reads (the 20 B/edge union estimate)
+      // per vertex: degree, bucket, first words, two labels
+      ProfScope prof(stream, "k_cc_sample", kSampleSteps * 40.0 * g->n);
+      auto hook = g->weighted ? k_cc_hook<true> : k_cc_hook<false>;
+      auto sample = g->weighted ? k_cc_sample<true> : k_cc_sample<false>;
+      for (uint32_t step = 0; step < kSampleSteps; ++step) {
+        if (step == 0)
+          hook<<<unsigned((uint64_t(g->n) + kHookBlock - 1) / kHookBlock), kHookBlock, 0,
+                 stream>>>(g->view(), parent);
+        else
+          sample<<<blocks_for_threads(g->n), kBlock, 0, stream>>>(g->view(), parent,
+                                                                  step == 1 ? 0 : 32);
+        k_cc_shorten<<<blocks_for_threads(g->n), kBlock, 0, stream>>>(parent, g->n);
+      }
+    }
+    {
+      // per bucket: owner + degree (8 B) and its slabs; per edge one label
       uint64_t m = 0;
       if (profiling_on()) (void)mk_graph_num_edges(g, &m);
-      ProfScope prof(stream, "k_cc_edges", 264.0 * g->total_buckets + 20.0 * double(m));
+      ProfScope prof(stream, "k_cc_edges", 264.0 * g->total_buckets + 4.0 * double(m));
       if (g->weighted)
         k_cc_edges<true><<<grid, kBlock, 0, stream>>>(g->view(), parent);
       else

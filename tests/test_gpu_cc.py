@@ -69,3 +69,26 @@ def test_directed_graph_weak_components(gpu):
     cc.Incremental(np.array([15], np.uint32), np.array([12], np.uint32))
     lab = cc.Labels()
     assert lab[15] == 12 and lab[12] == 12
+
+
+@pytest.mark.parametrize("weighted,hints", [(False, True), (True, True), (False, False)])
+def test_static_over_tombstones_and_chains(gpu, weighted, hints):
+    # the words a vertex is first joined by deleted, several buckets or long
+    # chains a vertex, edges held in one direction only, a last vertex alone
+    n, s, d, w = gen.rmat(13, 3, seed=17, weighted=True)
+    n += 1
+    pool = mk.SlabPool(1 << 26)
+    g = mk.DynamicGraph(n, pool, 0.7, gen.degree_hints(n, s) if hints else None,
+                        weighted=weighted)
+    g.InsertEdges(s, d, w if weighted else None)
+    cc = mk.CC(g)
+    keys = gen.keys_of(s, d)
+    for i in range(3):
+        cc.Static()
+        s2, d2 = gen.split_keys(keys)
+        both = np.unique(np.r_[gen.keys_of(s2, d2), gen.keys_of(d2, s2)])
+        want = oracle.cc(oracle.csr(n, *gen.split_keys(both)))[0]
+        assert np.array_equal(cc.Labels(), want), i
+        gone = gen.delete_batch(keys, len(keys) // 2, seed=90 + i)
+        g.DeleteEdges(*gone)
+        keys = keys[~np.isin(keys, gen.keys_of(*gone))]
