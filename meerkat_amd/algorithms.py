@@ -44,13 +44,18 @@ class _Traversal:
 
     def read(self):
         """(distances, parents) as uint32 numpy arrays; INF = 0xFFFFFFFF."""
-        d = np.empty(self.G.n, np.uint32)
-        p = np.empty(self.G.n, np.uint32)
-        _lib.call(f"{self._prefix}_read", self._h, d.ctypes.data_as(_vp), p.ctypes.data_as(_vp))
+        return self._read(True, True)
+
+    def _read(self, dist, parents):
+        """The wanted arrays (None for the other): each is a transfer of its own."""
+        d = np.empty(self.G.n, np.uint32) if dist else None
+        p = np.empty(self.G.n, np.uint32) if parents else None
+        _lib.call(f"{self._prefix}_read", self._h, None if d is None else d.ctypes.data_as(_vp),
+                  None if p is None else p.ctypes.data_as(_vp))
         return d, p
 
     def Distances(self):
-        return self.read()[0]
+        return self._read(True, False)[0]
 
     def capture_step(self, del_src, del_dst, ins_src, ins_dst, ins_w=None):
         """Record one update step on fixed device batch buffers (torch
@@ -72,7 +77,7 @@ class _Traversal:
         return CapturedStep(out, bufs)
 
     def Parents(self):
-        return self.read()[1]
+        return self._read(False, True)[1]
 
     def set_deferred(self, on=True):
         """Deferred calls: Incremental / Decremental return once queued on the

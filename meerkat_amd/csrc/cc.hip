@@ -22,6 +22,7 @@
 #include <algorithm>
 
 #include "profile.hpp"
+#include "readback.hpp"
 #include "slabhash.hpp"
 
 namespace mk {
@@ -354,9 +355,7 @@ int mk_cc_decremental(mk_cc *c, const uint32_t *src, const uint32_t *dst, uint32
 int mk_cc_labels(mk_cc *c, uint32_t *labels) {
   if (!c || !labels) return fail(MK_ERR_BAD_ARG, "mk_cc_labels: NULL argument");
   MK_HIP(hipSetDevice(c->c.g->device));
-  MK_HIP(hipStreamSynchronize(c->c.stream));
-  MK_HIP(hipMemcpy(labels, c->c.parent, size_t(c->c.g->n) * 4, hipMemcpyDeviceToHost));
-  return MK_OK;
+  return read_words(labels, c->c.g->n, c->c.g->device, c->c.stream, WordsOf{c->c.parent});
 }
 
 }  // extern "C"

@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "profile.hpp"
+#include "readback.hpp"
 #include "slabhash.hpp"
 
 namespace mk {
@@ -615,11 +616,6 @@ __global__ void __launch_bounds__(64) k_ms_admit(GraphView G, MsView S, MsAdmit 
   push_hubs(G, S.ql[qs], &S.c->large[qs], hub, v, nb);
 }
 
-__global__ void k_mssp_read(const uint32_t *dist, uint32_t n, uint32_t s, uint32_t *out) {
-  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < n) out[v] = dist[size_t(v) * 64 + s];
-}
-
 // ------------------------------------------------------------------ host
 struct MultiSource {
   mk_graph *g = nullptr;
@@ -638,6 +634,7 @@ struct MultiSource {
   uint32_t *src_dev = nullptr;
   uint32_t *off = nullptr;  // BFS: admission level per slot
   HostBuf host;
+  DevBuf read_buf;          // BFS: one slot's distances, scattered from the log
   // continuous batching (open / admit / launch / poll): the session's next
   // step, the slots admitted since open, and whether a session is open
   bool session = false;
@@ -734,6 +731,7 @@ struct MultiSource {
     (void)hipFree(c);
     (void)hipFree(src_dev);
     (void)hipFree(off);
+    read_buf.release();
     host.release();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -935,9 +933,9 @@ struct MultiSource {
       return fail(MK_ERR_RANGE, session ? "mk_msq_read: slot not admitted in this session"
                                         : "mk_msq_read: slot not in the last run");
     MK_HIP(hipSetDevice(g->device));
-    DevBuf b;
-    if (int r = b.ensure(size_t(g->n) * 4)) return r;
-    if (session && !sssp) {
+    if (sssp) return read_words(out, g->n, g->device, stream, ColumnOf{dist, slot});
+    if (int r = read_buf.ensure(size_t(g->n) * 4)) return r;
+    if (session) {
       // the log so far: levels 0 .. step - 1 are written
       uint32_t total = 0;
       MK_HIP(hipMemcpyAsync(&total, seg + step, 4, hipMemcpyDeviceToHost, stream));
@@ -945,20 +943,11 @@ struct MultiSource {
       log_total = std::min(total, log_cap);
       last_steps = step;
     }
-    if (sssp) {
-      k_mssp_read<<<blocks_for_threads(g->n), kBlock, 0, stream>>>(dist, g->n, slot,
-                                                                   b.as<uint32_t>());
-    } else {
-      fill_u32(b.as<uint32_t>(), kInf, g->n, stream);
-      if (log_total)
-        k_msbfs_read<<<blocks_for_threads(log_total), kBlock, 0, stream>>>(
-            view(), slot, log_total, last_steps + 1, b.as<uint32_t>());
-    }
-    hipError_t e = hipStreamSynchronize(stream);
-    if (e == hipSuccess) e = hipMemcpy(out, b.ptr, size_t(g->n) * 4, hipMemcpyDeviceToHost);
-    b.release();
-    if (e != hipSuccess) return hip_fail(e, "mk_msq_read");
-    return MK_OK;
+    fill_u32(read_buf.as<uint32_t>(), kInf, g->n, stream);
+    if (log_total)
+      k_msbfs_read<<<blocks_for_threads(log_total), kBlock, 0, stream>>>(
+          view(), slot, log_total, last_steps + 1, read_buf.as<uint32_t>());
+    return read_words(out, g->n, g->device, stream, WordsOf{read_buf.as<uint32_t>()});
   }
 };
 

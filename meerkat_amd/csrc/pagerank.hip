@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "profile.hpp"
+#include "readback.hpp"
 #include "slabhash.hpp"
 
 namespace mk {
@@ -901,9 +902,8 @@ struct PageRank {
 
   int read(float *out) {
     MK_HIP(hipSetDevice(g->device));
-    MK_HIP(hipStreamSynchronize(stream));
-    MK_HIP(hipMemcpy(out, pr[cur], size_t(g->n) * 4, hipMemcpyDeviceToHost));
-    return MK_OK;
+    return read_words(reinterpret_cast<uint32_t *>(out), g->n, g->device, stream,
+                      WordsOf{reinterpret_cast<const uint32_t *>(pr[cur])});
   }
 };
 

@@ -42,6 +42,7 @@
 #include <vector>
 
 #include "profile.hpp"
+#include "readback.hpp"
 #include "slabhash.hpp"
 
 namespace mk {
@@ -1631,14 +1632,6 @@ __global__ void k_set_source(GraphView G, uint64_t *dist, uint32_t source, uint3
   }
 }
 
-__global__ void k_unpack(const uint64_t *dist, uint32_t n, uint32_t *d, uint32_t *p) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint64_t x = dist[i];
-  if (d) d[i] = dist_of(x);
-  if (p) p[i] = parent_of(x);
-}
-
 // ---------------------------------------------------------------- host
 // Streams of the library's handles, per device (BFS/SSSP handles share
 // their graph's stream; multi-source, PageRank, TC and CC handles have their
@@ -2512,24 +2505,11 @@ struct Traversal {
   int read(uint32_t *d, uint32_t *p) {
     MK_HIP(hipSetDevice(g->device));
     if (int r = settle()) return r;
-    DevBuf b;
-    if (int r = b.ensure(size_t(g->n) * 8)) return r;
-    const int r = unpack_to_host(b.as<uint32_t>(), d, p);
-    b.release();
-    return r;
-  }
-
-  // Distances and parents unpacked into `staging` (2n words of device
-  // memory) on the handle's stream, then copied to the host.
-  int unpack_to_host(uint32_t *staging, uint32_t *d, uint32_t *p) {
-    const size_t n = g->n;
-    uint32_t *dd = staging, *pp = staging + n;
-    k_unpack<<<blocks_for_threads(n), kBlock, 0, stream>>>(dist, g->n, dd, pp);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && d) e = hipMemcpyAsync(d, dd, n * 4, hipMemcpyDeviceToHost, stream);
-    if (e == hipSuccess && p) e = hipMemcpyAsync(p, pp, n * 4, hipMemcpyDeviceToHost, stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
-    if (e != hipSuccess) return hip_fail(e, "read distances");
+    if (d)
+      if (int r = read_words(d, g->n, g->device, stream, HighOf{dist})) return r;
+    if (p)
+      if (int r = read_words(p, g->n, g->device, stream, LowOf{dist})) return r;
+    MK_HIP(hipStreamSynchronize(stream));
     return MK_OK;
   }
 };
