@@ -167,11 +167,12 @@ MK_DEV void push_hubs(const GraphView &G, uint2 *queue, unsigned long long *coun
     }
   }
   const uint32_t leader = ffs64(hm);
+  // lane 63's sums are read with every lane active: a sum used in the
+  // leader's branch only may be computed there, by the leader alone
+  const uint32_t total = read_lane(xc, 63), buckets = read_lane(xb, 63);
   unsigned long long r = 0;
-  if (lane == leader)
-    r = atomicAdd(count, (uint64_t(read_lane(xc, 63)) << 32) | read_lane(xb, 63));
+  if (lane == leader) r = atomicAdd(count, (uint64_t(total) << 32) | buckets);
   const uint32_t first = read_lane(uint32_t(r >> 32), leader);
-  const uint32_t total = read_lane(xc, 63);
   const uint32_t b0 = hub ? G.bucket_off[v] : 0u;
   // the wave writes the entries together, 64 at a time: entry e belongs to
   // the first lane whose inclusive prefix exceeds e (found by halving)

@@ -220,7 +220,8 @@ __global__ void __launch_bounds__(kBlock)
       for (uint32_t k = 0; k < kPrBatch; ++k) {
         if (k >= c) continue;
         const float s = chain_sum<MAP>(R, contrib, x[k], slabs);
-        if (lane == 0) atomicAdd(&P.hub_acc[read_lane(h, js[k])], double(s));
+        const uint32_t hk = read_lane(h, js[k]);  // with every lane active
+        if (lane == 0) atomicAdd(&P.hub_acc[hk], double(s));
       }
     }
   }

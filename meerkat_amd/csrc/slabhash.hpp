@@ -135,6 +135,19 @@ MK_DEV void load_words(const uint32_t *p, uint32_t (&v)[kWordsPerLane]) {
     v[4 * k + 3] = x.w;
   }
 }
+// load_words for words that are read once: past the caches' reuse order.
+MK_DEV void load_words_once(const uint32_t *p, uint32_t (&v)[kWordsPerLane]) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const u32x4 *q = reinterpret_cast<const u32x4 *>(p);
+#pragma unroll
+  for (uint32_t k = 0; k < kWordsPerLane / 4; ++k) {
+    const u32x4 x = __builtin_nontemporal_load(q + k);
+    v[4 * k] = x.x;
+    v[4 * k + 1] = x.y;
+    v[4 * k + 2] = x.z;
+    v[4 * k + 3] = x.w;
+  }
+}
 // v[j] for a lane-varying j (a select chain, no scratch indexing).
 MK_DEV uint32_t pick(const uint32_t (&v)[kWordsPerLane], uint32_t j) {
   uint32_t r = v[0];

@@ -242,11 +242,30 @@ struct TravView {
   uint2 *far[3];
   uint32_t far_cap;
   uint32_t delta;
+  // Dense steps of a static run (bound == nullptr: other calls, none).
+  // `bound`: upper bounds of the distances in 16 bits (kNoBound: none
+  // known), read in place of the 64-bit pairs: a quarter of their lines,
+  // most of which stay in L2.  Every improvement of the run stores its
+  // distance here; a bound that is out of date (stores that crossed, another
+  // XCD's copy) is only too high and lets an extra atomic through.
+  // `done`: a distance at or above each one that the vertex's edges were all
+  // relaxed with (kInf: none yet): a vertex whose distance has fallen below
+  // it has to be expanded again.
+  uint16_t *bound;
+  uint32_t *done;
   // added to every stamp epoch a kernel is given: zero for calls made
   // through the API, the replay's base while a captured update step
   // (mk_step) runs, so each replay stamps with epochs of its own
   const uint32_t *ep_base;
 };
+
+constexpr uint32_t kNoBound = 0xFFFFu;
+// A static run improved v to d and, with `queued`, queues it for that.
+MK_DEV void note_improved(const TravView &S, uint32_t v, uint32_t d, bool queued) {
+  if (!S.bound) return;
+  if (d < kNoBound) S.bound[v] = uint16_t(d);
+  if (queued) coherent_store(S.done + v, d);
+}
 
 MK_DEV uint32_t wave_min_u32(uint32_t x) {
   for (int off = 32; off >= 1; off >>= 1) {
@@ -298,7 +317,10 @@ MK_DEV void enqueue_nb(const GraphView &G, const TravView &S, WaveQ &q, uint32_t
 
 // Bucket count of v for the lanes that push it (0 elsewhere).
 MK_DEV uint32_t push_buckets(const GraphView &G, bool push, uint32_t v) {
-  return push ? G.bucket_off[v + 1] - G.bucket_off[v] : 0u;
+  if (!push) return 0u;
+  uint32_t o[2];
+  __builtin_memcpy(o, G.bucket_off + v, 8);  // one load, 4-byte aligned
+  return o[1] - o[0];
 }
 
 MK_DEV void enqueue(const GraphView &G, const TravView &S, WaveQ &q, uint32_t side,
@@ -451,7 +473,10 @@ MK_DEV uint32_t slab_work(const GraphView &G, const TravView &S, Sink &sink, uin
       if (D >= du && D < dist_of(S.dist[v])) {
         const uint64_t old = atomicMin((unsigned long long *)(S.dist + v),
                                        (unsigned long long)pack(D, u));
-        if (D < dist_of(old)) push = atomicExch(S.stamp + v, epoch) != epoch;
+        if (D < dist_of(old)) {
+          push = atomicExch(S.stamp + v, epoch) != epoch;
+          note_improved(S, v, D, push);
+        }
       }
     }
   } else if (MODE == 1) {  // invalidate tree children of u
@@ -494,11 +519,9 @@ MK_DEV void chain_work(const GraphView &G, const TravView &S, Sink &sink, uint32
 }
 
 // slab_work over c <= kBatch slabs at once (slab k of vertex u[k] with
-// distance du[k], this lane's word v[k]), phase by phase, so that the
-// dependent memory operations of the slabs overlap instead of following
-// one another: every distance (invalid bit) load, then every atomic (with
-// the bucket count of each candidate vertex), then every stamp (bitmap)
-// update, then the pushes.  Wave-collective; returns live keys seen.
+// distance du[k], this lane's word v[k]), phase by phase (as
+// group_slab_work): a key per lane, the fewest instructions for the few
+// slabs a wave has in a small step.  Wave-collective; returns live keys seen.
 template <bool MAP, bool WEIGHTS, int MODE, typename Sink>
 MK_DEV uint32_t batch_slab_work(const GraphView &G, const TravView &S, Sink &sink, uint32_t epoch,
                                 uint32_t c, const uint32_t (&u)[kBatch],
@@ -548,6 +571,7 @@ MK_DEV uint32_t batch_slab_work(const GraphView &G, const TravView &S, Sink &sin
       if (push[k]) atomicOr(S.invbits + (v[k] >> 5), 1u << (v[k] & 31u));
     } else if (push[k]) {
       push[k] = atomicExch(S.stamp + v[k], epoch) != epoch;
+      if (MODE == 0) note_improved(S, v[k], D[k], push[k]);
     }
   }
   uint32_t edges = 0;
@@ -559,47 +583,259 @@ MK_DEV uint32_t batch_slab_work(const GraphView &G, const TravView &S, Sink &sin
   return edges;
 }
 
-// Process the buckets named by lanes of `m`: lane j owns bucket bk (its
-// vertex uj with distance dj).  Head slabs are loaded and worked kBatch at
-// a time (batch_slab_work); chained slabs follow one by one.
+// Lane of the r-th lowest set bit of m in lane r (r < popcount): a lane-wide
+// gather from there packs the lanes of m to the front.  Wave-collective.
+MK_DEV uint32_t pack_lanes(uint64_t m) {
+  const uint32_t lane = lane_id();
+  const bool in = (m >> lane) & 1ull;
+  const uint32_t at = in ? lanes_below(m) : uint32_t(__popcll(m)) + lanes_below(~m);
+  return uint32_t(__builtin_amdgcn_ds_permute(int(at * 4), int(lane)));
+}
+
+// Work of the three passes on one slab per 8-lane group (group's vertex u
+// with distance du, its lane's eight slab words w; `has`: the group has a
+// slab), phase by phase, so that the dependent memory operations of all
+// keys of the eight slabs overlap: every distance (invalid bit) load, then
+// every atomic (with the bucket count of each candidate vertex), then every
+// stamp (bitmap) update, then the pushes.  Wave-collective; returns live
+// keys seen (over the wave).
 template <bool MAP, bool WEIGHTS, int MODE, typename Sink>
+MK_DEV uint32_t group_slab_work(const GraphView &G, const TravView &S, Sink &sink, uint32_t epoch,
+                                bool has, uint32_t u, uint32_t du,
+                                const uint32_t (&w)[kWordsPerLane]) {
+  constexpr uint32_t kStep = MAP ? 2 : 1, kKeys = kWordsPerLane / kStep;
+  const uint32_t gl = group_lane();
+  bool live[kKeys], ok[kKeys];
+  uint32_t D[kKeys];
+  uint64_t cur[kKeys];
+#pragma unroll
+  for (uint32_t k = 0; k < kKeys; ++k) {
+    const uint32_t v = w[k * kStep];
+    live[k] = has && key_word<MAP>(kWordsPerLane * gl + k * kStep) && v < kTomb;
+    D[k] = du + (WEIGHTS ? w[k * kStep + (MAP ? 1 : 0)] : 1u);
+    ok[k] = live[k] && (MODE == 1 || D[k] >= du);
+    cur[k] = kInfInf;
+    if (MODE == 2) {
+      if (ok[k]) ok[k] = inv_bit(S.invbits, v);
+    } else if (ok[k]) {
+      // MODE 1: values only move to INF during this pass, so a plain load
+      // suffices; MODE 0: a stale value only lets an extra atomic through
+      cur[k] = S.dist[v];
+    }
+  }
+  uint32_t edges = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kKeys; ++k) edges += uint32_t(__popcll(ballot(live[k])));
+  // the atomics, with the bucket counts of their lanes loaded alongside
+  // (read only where the vertex is then pushed)
+  bool push[kKeys];
+  uint32_t nb[kKeys];
+#pragma unroll
+  for (uint32_t k = 0; k < kKeys; ++k) {
+    const uint32_t v = w[k * kStep];
+    push[k] = false;
+    const bool cand = MODE == 1 ? ok[k] && cur[k] != kInfInf && parent_of(cur[k]) == u
+                                : ok[k] && (MODE == 2 || D[k] < dist_of(cur[k]));
+    nb[k] = push_buckets(G, cand, v);
+    if (MODE == 1) {
+      if (cand)
+        push[k] = atomicCAS((unsigned long long *)(S.dist + v), (unsigned long long)cur[k],
+                            (unsigned long long)kInfInf) == cur[k];
+    } else if (cand) {
+      cur[k] = atomicMin((unsigned long long *)(S.dist + v), (unsigned long long)pack(D[k], u));
+      push[k] = D[k] < dist_of(cur[k]);  // improved
+    }
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < kKeys; ++k) {
+    const uint32_t v = w[k * kStep];
+    if (MODE == 1) {
+      if (push[k]) atomicOr(S.invbits + (v >> 5), 1u << (v & 31u));
+    } else if (push[k]) {
+      push[k] = atomicExch(S.stamp + v, epoch) != epoch;
+      if (MODE == 0) note_improved(S, v, D[k], push[k]);
+    }
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < kKeys; ++k) sink(G, push[k], w[k * kStep], nb[k]);
+  return edges;
+}
+
+// Process the buckets named by lanes of `m`: lane j owns bucket bk (its
+// vertex uj with distance dj).  Eight buckets at a time, one per 8-lane
+// group, their head slabs loaded together and the next eight's in flight;
+// chained slabs follow, the groups that have one together (static SSSP on
+// RMAT-24: 17.3 ms with a slab a wave throughout, 14.2 in groups).  Set
+// slabs, eight key words a lane, are worked in groups only where a wave has
+// many nearly empty ones: a hub's (HUB) are full, a key for nearly every
+// lane (BFS on RMAT-16: its hub step 32 us so, 72 us in groups), and up to
+// kBatch slabs take fewer instructions that way (BFS over a 1M-vertex grid,
+// a vertex a wave: 14.9 ms, 17.0 in groups).
+template <bool MAP, bool WEIGHTS, int MODE, bool HUB, typename Sink>
 MK_DEV void batched_buckets(const GraphView &G, const TravView &S, Sink &sink, uint32_t epoch,
                             uint64_t m, uint32_t bk, uint32_t uj, uint32_t dj, uint32_t &slabs,
                             uint32_t &edges) {
-  const uint32_t lane = lane_id();
-  while (m) {
-    uint32_t js[kBatch];
-    uint32_t c = 0;
+  if (m == 0) return;
+  const uint32_t n = uint32_t(__popcll(m));
+  if (!MAP && (HUB || n <= kBatch)) {
+    const uint32_t lane = lane_id();
+    while (m) {
+      uint32_t v[kBatch], us[kBatch], ds[kBatch], c = 0;
 #pragma unroll
-    for (uint32_t k = 0; k < kBatch; ++k) {
-      js[k] = m ? ffs64(m) : 0u;
-      if (m) {
-        m &= m - 1;
-        c = k + 1;
+      for (uint32_t k = 0; k < kBatch; ++k) {
+        const uint32_t j = m ? ffs64(m) : 0u;
+        v[k] = m ? G.heads[size_t(read_lane(bk, j)) * kSlabWords + lane] : kEmpty;
+        us[k] = read_lane(uj, j);
+        ds[k] = read_lane(dj, j);
+        if (m) {
+          m &= m - 1;
+          c = k + 1;
+        }
+      }
+      slabs += c;
+      edges += batch_slab_work<MAP, WEIGHTS, MODE>(G, S, sink, epoch, c, us, ds, v);
+#pragma unroll
+      for (uint32_t k = 0; k < kBatch; ++k) {
+        const uint32_t nx = k < c ? read_lane(v[k], kNextLane) : kEmpty;
+        if (nx != kEmpty)
+          chain_work<MAP, WEIGHTS, MODE>(G, S, sink, epoch, us[k], ds[k],
+                                         slab_ptr(G.pool, nx)[lane], slabs, edges);
       }
     }
-    uint32_t v[kBatch], us[kBatch], ds[kBatch];
+    return;
+  }
+  const uint32_t gl = group_lane(), grp = lane_id() / kGroupLanes;
+  const uint32_t from = pack_lanes(m);
+  const uint32_t bp = uint32_t(__shfl(int(bk), int(from), 64));
+  const uint32_t up = uint32_t(__shfl(int(uj), int(from), 64));
+  const uint32_t dp = uint32_t(__shfl(int(dj), int(from), 64));
+  uint32_t nxt[kWordsPerLane];
+  uint32_t bn = uint32_t(__shfl(int(bp), int(grp), 64));
+  if (grp < n) load_words(G.heads + size_t(bn) * kSlabWords + kWordsPerLane * gl, nxt);
+  for (uint32_t i = 0; i < n; i += kGroupsPerWave) {
+    uint32_t w[kWordsPerLane];
 #pragma unroll
-    for (uint32_t k = 0; k < kBatch; ++k) {
-      v[k] = k < c ? G.heads[size_t(read_lane(bk, js[k])) * kSlabWords + lane] : kEmpty;
-      us[k] = read_lane(uj, js[k]);
-      ds[k] = read_lane(dj, js[k]);
+    for (uint32_t k = 0; k < kWordsPerLane; ++k) w[k] = nxt[k];
+    bool has = i + grp < n;
+    const uint32_t u = uint32_t(__shfl(int(up), int(i + grp), 64));
+    const uint32_t du = uint32_t(__shfl(int(dp), int(i + grp), 64));
+    const uint32_t in = i + kGroupsPerWave + grp;
+    bn = uint32_t(__shfl(int(bp), int(in & 63u), 64));
+    if (in < n) load_words(G.heads + size_t(bn) * kSlabWords + kWordsPerLane * gl, nxt);
+    for (;;) {
+      slabs += uint32_t(__popcll(ballot(has && gl == 0)));
+      edges += group_slab_work<MAP, WEIGHTS, MODE>(G, S, sink, epoch, has, u, du, w);
+      const uint32_t nx = group_read(w[kWordsPerLane - 1], kGroupLanes - 1);
+      has = has && nx != kEmpty;
+      if (ballot(has) == 0) break;
+      if (has) load_words(slab_ptr(G.pool, nx) + kWordsPerLane * gl, w);
     }
-    slabs += c;
-    edges += batch_slab_work<MAP, WEIGHTS, MODE>(G, S, sink, epoch, c, us, ds, v);
+  }
+}
+
+// Dense relax of the buckets named by lanes of `m` (as batched_buckets):
+// improved vertices get the step's epoch as their stamp (collect_step finds
+// them), by stores and atomics that nothing waits for, kDenseSlabs buckets
+// per 8-lane group at a time (their distance loads in flight together) and
+// the next ones' slabs on their way.
+MK_DEV void load_words_nt(const uint32_t *p, uint32_t (&v)[kWordsPerLane]) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  const u4 *q = reinterpret_cast<const u4 *>(p);
 #pragma unroll
-    for (uint32_t k = 0; k < kBatch; ++k) {
-      const uint32_t nx = k < c ? read_lane(v[k], kNextLane) : kEmpty;
-      if (nx != kEmpty)
-        chain_work<MAP, WEIGHTS, MODE>(G, S, sink, epoch, us[k], ds[k],
-                                       slab_ptr(G.pool, nx)[lane], slabs, edges);
+  for (uint32_t k = 0; k < 2; ++k) { const u4 x = __builtin_nontemporal_load(q + k); v[4*k]=x.x; v[4*k+1]=x.y; v[4*k+2]=x.z; v[4*k+3]=x.w; }
+}
+template <bool MAP, bool WEIGHTS, bool HUB>
+MK_DEV void dense_buckets(const GraphView &G, const TravView &S, uint64_t m, uint32_t bk,
+                          uint32_t uj, uint32_t dj, uint32_t &slabs, uint32_t &edges) {
+  if (m == 0) return;
+  if (!MAP && HUB) {  // full set slabs: a key per lane, kBatch slabs at a time
+    const uint32_t lane = lane_id();
+    while (m) {
+      uint32_t v[kBatch], most[kBatch], us[kBatch], D[kBatch];
+      bool more = false;
+#pragma unroll
+      for (uint32_t k = 0; k < kBatch; ++k) {
+        const uint32_t j = m ? ffs64(m) : 0u;
+        v[k] = m ? G.heads[size_t(read_lane(bk, j)) * kSlabWords + lane] : kEmpty;
+        slabs += m ? 1u : 0u;
+        us[k] = read_lane(uj, j);
+        D[k] = read_lane(dj, j) + 1u;
+        m &= m - 1;
+      }
+      do {
+#pragma unroll
+        for (uint32_t k = 0; k < kBatch; ++k) {
+          const bool live = lane != kNextLane && v[k] < kTomb;
+          edges += uint32_t(__popcll(ballot(live)));
+          most[k] = live ? S.bound[v[k]] : 0u;
+        }
+        more = false;
+#pragma unroll
+        for (uint32_t k = 0; k < kBatch; ++k) {
+          if (D[k] != 0u && (D[k] < most[k] || most[k] == kNoBound)) {
+            (void)atomicMin((unsigned long long *)(S.dist + v[k]),
+                            (unsigned long long)pack(D[k], us[k]));
+            if (D[k] < kNoBound) S.bound[v[k]] = uint16_t(D[k]);
+          }
+          const uint32_t nx = read_lane(v[k], kNextLane);
+          v[k] = nx != kEmpty ? slab_ptr(G.pool, nx)[lane] : kEmpty;
+          slabs += nx != kEmpty ? 1u : 0u;
+          more |= nx != kEmpty;
+        }
+      } while (more);
+    }
+    return;
+  }
+  constexpr uint32_t kStep = MAP ? 2 : 1, kKeys = kWordsPerLane / kStep;
+  const uint32_t gl = group_lane(), grp = lane_id() / kGroupLanes;
+  const uint32_t n = uint32_t(__popcll(m));
+  const uint32_t from = pack_lanes(m);
+  const uint32_t bp = uint32_t(__shfl(int(bk), int(from), 64));
+  const uint32_t up = uint32_t(__shfl(int(uj), int(from), 64));
+  const uint32_t dp = uint32_t(__shfl(int(dj), int(from), 64));
+  uint32_t nxt[kWordsPerLane];
+  uint32_t bn = uint32_t(__shfl(int(bp), int(grp), 64));
+  if (grp < n) load_words_once(G.heads + size_t(bn) * kSlabWords + kWordsPerLane * gl, nxt);
+  for (uint32_t i = 0; i < n; i += kGroupsPerWave) {
+    uint32_t w[kWordsPerLane];
+#pragma unroll
+    for (uint32_t k = 0; k < kWordsPerLane; ++k) w[k] = nxt[k];
+    bool has = i + grp < n;
+    const uint32_t u = uint32_t(__shfl(int(up), int(i + grp), 64));
+    const uint32_t du = uint32_t(__shfl(int(dp), int(i + grp), 64));
+    const uint32_t in = i + kGroupsPerWave + grp;
+    bn = uint32_t(__shfl(int(bp), int(in & 63u), 64));
+    if (in < n) load_words_once(G.heads + size_t(bn) * kSlabWords + kWordsPerLane * gl, nxt);
+    for (;;) {
+      slabs += uint32_t(__popcll(ballot(has && gl == 0)));
+      uint32_t most[kKeys];  // a dead key: 0, which nothing is below
+#pragma unroll
+      for (uint32_t k = 0; k < kKeys; ++k) {
+        const uint32_t v = w[k * kStep];
+        const bool live = has && key_word<MAP>(kWordsPerLane * gl + k * kStep) && v < kTomb;
+        edges += uint32_t(__popcll(ballot(live)));
+        most[k] = live ? S.bound[v] : 0u;
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < kKeys; ++k) {
+        const uint32_t v = w[k * kStep];
+        const uint32_t D = du + (WEIGHTS ? w[k * kStep + (MAP ? 1 : 0)] : 1u);
+        if (D >= du && (D < most[k] || most[k] == kNoBound)) {
+          (void)atomicMin((unsigned long long *)(S.dist + v), (unsigned long long)pack(D, u));
+          if (D < kNoBound) S.bound[v] = uint16_t(D);
+        }
+      }
+      const uint32_t nx = group_read(w[kWordsPerLane - 1], kGroupLanes - 1);
+      has = has && nx != kEmpty;
+      if (ballot(has) == 0) break;
+      if (has) load_words_once(slab_ptr(G.pool, nx) + kWordsPerLane * gl, w);
     }
   }
 }
 
 // Expand frontier vertices queue[0..n) (non-hub entries), waves wave,
 // wave + NW, ... of the caller taking up to 64 each.
-template <bool MAP, bool WEIGHTS, int MODE, typename Sink>
+template <bool MAP, bool WEIGHTS, int MODE, bool DENSE = false, typename Sink>
 MK_DEV void expand_rows(const GraphView &G, const TravView &S, Sink &sink, uint32_t epoch,
                         const uint32_t *queue, uint32_t n, uint32_t wave, uint32_t NW,
                         uint32_t &slabs, uint32_t &edges, uint32_t &visited, uint32_t T = kInf,
@@ -622,11 +858,16 @@ MK_DEV void expand_rows(const GraphView &G, const TravView &S, Sink &sink, uint3
       if (S.delta && far_append(S, fcur, act && du >= T, u, du)) act = false;
     }
     visited += uint32_t(__popcll(ballot(act)));
-    batched_buckets<MAP, WEIGHTS, MODE>(G, S, sink, epoch, ballot(act), b0, u, du, slabs, edges);
-    // further buckets (at most kSmallBuckets - 1 for queued vertices)
-    for (uint32_t k = 1; ballot(act && nb > k); ++k)
-      batched_buckets<MAP, WEIGHTS, MODE>(G, S, sink, epoch, ballot(act && nb > k), b0 + k, u,
-                                          du, slabs, edges);
+    // one lane expands all of the vertex, with this distance
+    if (MODE == 0 && S.bound && act) coherent_store(S.done + u, du);
+    // at most kSmallBuckets buckets for queued vertices
+    for (uint32_t k = 0; ballot(act && nb > k); ++k)
+      if constexpr (DENSE)
+        dense_buckets<MAP, WEIGHTS, false>(G, S, ballot(act && nb > k), b0 + k, u, du, slabs,
+                                           edges);
+      else
+        batched_buckets<MAP, WEIGHTS, MODE, false>(G, S, sink, epoch, ballot(act && nb > k),
+                                                   b0 + k, u, du, slabs, edges);
   }
 }
 
@@ -704,7 +945,15 @@ constexpr uint32_t kWideWaveLds = (kWideBlock / 64) * kWaveQ + kWideBlock / 64 +
 constexpr uint32_t kLoopLds = 2 * kTailCap + 4 > kWideWaveLds ? 2 * kTailCap + 4 : kWideWaveLds;
 constexpr uint32_t kExpandLds = 2 * kTailCap + 4 > kWaveLds ? 2 * kTailCap + 4 : kWaveLds;
 
-template <bool MAP, bool WEIGHTS, int MODE>
+// A static run's relax step whose frontier holds more than 1/kDenseShare of
+// the graph's buckets is dense: it improves so many vertices, most of them
+// more than once, that finding them by one pass over all vertices costs less
+// than a returning atomic, a stamp exchange, a bucket count and a queue entry
+// per improvement.
+constexpr uint32_t kDenseShare = 128;
+constexpr uint32_t kDenseLeast = 16384;  // and at least this many buckets
+
+template <bool MAP, bool WEIGHTS, int MODE, bool DENSE = false>
 MK_DEV void expand_step(const GraphView &G, const TravView &S, uint32_t side, uint32_t slot,
                         uint32_t epoch, uint32_t *lds, uint32_t T = kInf, uint32_t fcur = 0) {
   const uint32_t lane = lane_id();
@@ -723,7 +972,7 @@ MK_DEV void expand_step(const GraphView &G, const TravView &S, uint32_t side, ui
     if (n_small + n_large) atomicAdd(&S.cnt->steps, 1u);
   }
   if (n_small + n_large == 0) return;
-  if (n_large == 0 && n_small <= S.tail_enter) {
+  if (!DENSE && n_large == 0 && n_small <= S.tail_enter) {
     if (blockIdx.x == 0)
       expand_tail<MAP, WEIGHTS, MODE>(G, S, side, slot, epoch, n_small, lds, T, fcur);
     return;
@@ -763,18 +1012,57 @@ MK_DEV void expand_step(const GraphView &G, const TravView &S, uint32_t side, ui
         if (first && !stored) atomicExch(&S.cnt->far_over, 1u);
       }
     }
-    batched_buckets<MAP, WEIGHTS, MODE>(G, S, sink, epoch, ballot(act), b, u, du, slabs, edges);
+    if constexpr (DENSE)
+      dense_buckets<MAP, WEIGHTS, true>(G, S, ballot(act), b, u, du, slabs, edges);
+    else
+      batched_buckets<MAP, WEIGHTS, MODE, true>(G, S, sink, epoch, ballot(act), b, u, du, slabs,
+                                                edges);
   }
   // small vertices: up to 64 per wave step, spread over all waves when few
-  expand_rows<MAP, WEIGHTS, MODE>(G, S, sink, epoch, S.q_small[side], n_small, gw, W, slabs, edges,
-                                  visited, T, fcur);
-  block_flush(q, S.q_small[nside], &S.cnt->small[nslot], lds + (blockDim.x / 64) * kWaveQ);
+  expand_rows<MAP, WEIGHTS, MODE, DENSE>(G, S, sink, epoch, S.q_small[side], n_small, gw, W, slabs,
+                                         edges, visited, T, fcur);
+  if (!DENSE)
+    block_flush(q, S.q_small[nside], &S.cnt->small[nslot], lds + (blockDim.x / 64) * kWaveQ);
   if (lane == 0) {
     add_stat(S.cnt, MODE, kStatSlabs, slabs);
     add_stat(S.cnt, MODE, kStatEdges, edges);
     add_stat(S.cnt, MODE, kStatVisited, visited);
     add_stat(S.cnt, MODE, kStatPushed, q.pushed);
   }
+}
+
+// After a dense relax step (its grid barrier passed): every vertex whose
+// distance is below S.done is queued for the next one (queue side^1,
+// slot+1).  One pass over both arrays, four vertices a lane.  `lds` as
+// expand_step.
+MK_DEV void collect_step(const GraphView &G, const TravView &S, uint32_t side, uint32_t slot,
+                         uint32_t *lds) {
+  const uint32_t lane = lane_id();
+  const uint32_t gw = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const uint32_t W = (gridDim.x * blockDim.x) >> 6;
+  const uint32_t nslot = slot == 2 ? 0 : slot + 1;
+  const uint32_t nside = side ^ 1u;
+  WaveQ q{lds + (threadIdx.x >> 6) * kWaveQ, 0u, 0u};
+  GlobalSink sink{S, q, nside, nslot};
+  constexpr uint32_t kPer = 4;
+  for (uint64_t v0 = uint64_t(gw) * 64 * kPer; v0 < G.n; v0 += uint64_t(W) * 64 * kPer) {
+    uint32_t d[kPer], done[kPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+      const uint64_t v = v0 + k * 64 + lane;
+      d[k] = v < G.n ? dist_of(coherent_load64(S.dist + v)) : kInf;
+      done[k] = v < G.n ? coherent_load(S.done + v) : 0u;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+      const uint32_t v = uint32_t(v0) + k * 64 + lane;
+      const bool push = d[k] < done[k];
+      if (push) coherent_store(S.done + v, d[k]);
+      sink(G, push, v);
+    }
+  }
+  block_flush(q, S.q_small[nside], &S.cnt->small[nslot], lds + (blockDim.x / 64) * kWaveQ);
+  if (lane == 0) add_stat(S.cnt, kSetRelax, kStatPushed, q.pushed);
 }
 
 // One bottom-up step of a static BFS (no reference counterpart: the
@@ -1008,7 +1296,7 @@ __global__ void __launch_bounds__(kWideBlock)
   // cannot race with it
   const uint32_t bdone = coherent_load(&S.cnt->bar_done);
   if (S.trace && blockIdx.x == 0 && threadIdx.x == 0) S.cnt->loop_t[MODE][0] = wall_clock64();
-  uint32_t j = j0;
+  uint32_t j = j0, bars = 0;  // steps, grid barriers of this launch
   bool pulling = false;  // bottom-up steps (static BFS with the in-edge mirror)
   // near-far (static SSSP): the near bound and the number of splits so far,
   // as the launch this one continues left them
@@ -1046,7 +1334,7 @@ __global__ void __launch_bounds__(kWideBlock)
         }
       }
       if (!split) break;
-      if (!grid_barrier(S.bar, S.cnt, bdone + (j - j0) + 1, timeout, &flag)) return;
+      if (!grid_barrier(S.bar, S.cnt, bdone + ++bars, timeout, &flag)) return;
       continue;
     }
     if constexpr (MODE == 0 && !WEIGHTS) {
@@ -1058,11 +1346,23 @@ __global__ void __launch_bounds__(kWideBlock)
                           : fbuckets * S.pull_enter > G.total_buckets;
       }
     }
-    if (pulling)
+    bool dense = false;
+    if constexpr (MODE == 0)  // (near-far defers vertices that are then not done)
+      dense = !pulling && S.bound && !S.delta &&
+              (uint64_t(ns) + uint32_t(nl)) * kDenseShare > G.total_buckets &&
+              ns + uint32_t(nl) > kDenseLeast;
+    if (pulling) {
       pull_step<MAP>(G, S, j & 1u, slot, lds);
-    else
+    } else if (dense) {
+      if constexpr (MODE == 0) {
+        expand_step<MAP, WEIGHTS, MODE, true>(G, S, j & 1u, slot, ep, lds, T, nsplit % 3);
+        if (!grid_barrier(S.bar, S.cnt, bdone + ++bars, timeout, &flag)) return;
+        collect_step(G, S, j & 1u, slot, lds);
+      }
+    } else {
       expand_step<MAP, WEIGHTS, MODE>(G, S, j & 1u, slot, ep, lds, T, nsplit % 3);
-    if (!grid_barrier(S.bar, S.cnt, bdone + (j - j0) + 1, timeout, &flag)) return;
+    }
+    if (!grid_barrier(S.bar, S.cnt, bdone + ++bars, timeout, &flag)) return;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (S.trace) {
@@ -1073,7 +1373,7 @@ __global__ void __launch_bounds__(kWideBlock)
       S.cnt->loop_t[MODE][1] = now;
     }
     S.cnt->loop_end[MODE] = j;
-    S.cnt->bar_done = bdone + (j - j0);
+    S.cnt->bar_done = bdone + bars;
     if (MODE == 0 && S.delta) {
       S.cnt->nf_T = T;
       S.cnt->nf_split = nsplit;
@@ -1115,8 +1415,8 @@ __global__ void __launch_bounds__(kBlock)
       }
     }
     GlobalSink sink{S, q, 0u, 0u};
-    batched_buckets<MAP, WEIGHTS, 2>(G, S, sink, epoch, ballot(act), uint32_t(b), u, du, slabs,
-                                     edges);
+    batched_buckets<MAP, WEIGHTS, 2, false>(G, S, sink, epoch, ballot(act), uint32_t(b), u, du,
+                                            slabs, edges);
   }
   block_flush(q, S.q_small[0], &S.cnt->small[0], lq + (kBlock / 64) * kWaveQ);
   if (lane == 0) {
@@ -1618,8 +1918,13 @@ __global__ void __launch_bounds__(kBlock) k_repair(GraphView G, GraphView R, Tra
 // The source alone in the frontier of step 0 (queue side 0, slot 0), and
 // marked in `vbits0` (side 0's frontier bitmap) when bottom-up steps may run.
 __global__ void k_set_source(GraphView G, uint64_t *dist, uint32_t source, uint32_t *q_small,
-                             uint2 *q_large, Counts *cnt, uint32_t *vbits0) {
+                             uint2 *q_large, Counts *cnt, uint32_t *vbits0, uint16_t *bound,
+                             uint32_t *done) {
   dist[source] = pack(0, source);
+  if (bound) {
+    bound[source] = 0;
+    done[source] = 0;
+  }
   if (vbits0) vbits0[source >> 5] |= 1u << (source & 31u);
   const uint32_t b0 = G.bucket_off[source], nb = G.bucket_off[source + 1] - b0;
   if (nb <= kSmallBuckets) {
@@ -1686,6 +1991,9 @@ struct Traversal {
   bool repair = false;  // orphan repair before invalidation (with the in-edge mirror)
   bool persistent = true;        // frontier steps in one launch (k_expand_loop)
   uint32_t tail_enter = 128;     // tail-mode entry threshold (knob "tail_enter")
+  uint16_t *bound = nullptr;     // 16-bit distance bounds (static runs)
+  uint32_t *done = nullptr;      // distances expanded with (static runs)
+  bool bound_now = false;        // the launch being queued is a static run's
   uint32_t *vbits = nullptr;     // two frontier bitmaps (static BFS with the mirror)
   uint32_t pull_enter = 0, pull_exit = 1;  // knobs "pull_enter" / "pull_exit"
   bool pull_now = false;         // the launch being queued may take bottom-up steps
@@ -1727,6 +2035,8 @@ struct Traversal {
     v.far_cap = far_cap;
     v.delta = (delta_now && far[0]) ? delta : 0u;
     v.ep_base = ep_base;
+    v.bound = bound_now ? bound : nullptr;
+    v.done = done;
     return v;
   }
   uint32_t bit_words() const { return (g->n + 31) / 32; }
@@ -1746,6 +2056,8 @@ struct Traversal {
     MK_HIP(hipMalloc(&stamp, n * 4));
     MK_HIP(hipMalloc(&invbits, ((n + 31) / 32) * 4));
     MK_HIP(hipMalloc(&inv_list, n * 4));
+    MK_HIP(hipMalloc(&bound, (n + 1) / 2 * 4));
+    MK_HIP(hipMalloc(&done, n * 4));
     for (int i = 0; i < 2; ++i) {
       MK_HIP(hipMalloc(&qs[i], n * 4));
       // one entry per kHubChunk buckets of every listed hub (a vertex is
@@ -1766,7 +2078,8 @@ struct Traversal {
     fill_u32(stamp, 0u, n, stream);
     fill_u32(invbits, 0u, (n + 31) / 32, stream);
     clear_counts();
-    k_set_source<<<1, 1, 0, stream>>>(g->view(), dist, source, qs[0], ql[0], cnt, nullptr);
+    k_set_source<<<1, 1, 0, stream>>>(g->view(), dist, source, qs[0], ql[0], cnt, nullptr,
+                                      nullptr, nullptr);
     MK_HIP(hipStreamSynchronize(stream));
     max_waves = grid_waves(g->device);
     repair = tune_get("orphan_repair", 0) != 0;
@@ -1814,6 +2127,8 @@ struct Traversal {
     (void)hipFree(stamp);
     (void)hipFree(invbits);
     (void)hipFree(inv_list);
+    (void)hipFree(bound);
+    (void)hipFree(done);
     (void)hipFree(vbits);
     for (int i = 0; i < 3; ++i) (void)hipFree(far[i]);
     for (int i = 0; i < 2; ++i) {
@@ -2273,16 +2588,21 @@ struct Traversal {
     // a BFS over a graph with the in-edge mirror may take bottom-up steps
     pull_now = persistent && vbits != nullptr;
     if (pull_now) fill_u32(vbits, 0u, uint64_t(bit_words()) * 2, stream);
+    bound_now = persistent && !pull_now && (weights || g->total_buckets > (1u << 19));
+    if (bound_now) {
+      fill_u32(reinterpret_cast<uint32_t *>(bound), ~0u, (uint64_t(g->n) + 1) / 2, stream);
+      fill_u32(done, kInf, g->n, stream);
+    }
     // an SSSP with the knob sssp_delta set runs near-far (a loop that runs
     // out of steps is continued near-far too: end() relaunches it)
     delta_now = near_far && persistent && far[0] != nullptr;
     k_set_source<<<1, 1, 0, stream>>>(g->view(), dist, source, qs[0], ql[0], cnt,
-                                      pull_now ? vbits : nullptr);
+                                      pull_now ? vbits : nullptr, bound_now ? bound : nullptr, done);
     if (persistent) {
       const int r = queue_relax();
       pull_now = false;
       if (r) {
-        delta_now = false;
+        delta_now = bound_now = false;
         return r;
       }
     } else {
@@ -2291,7 +2611,7 @@ struct Traversal {
     }
     const bool nf = delta_now;
     const int r = end(ms);
-    delta_now = false;
+    delta_now = bound_now = false;
     // a deferred hub that found its far list full left buckets unexpanded:
     // the call is repeated without near-far
     if (r == MK_OK && nf && last_far_over) return run_static(ms, false);
