@@ -1426,151 +1426,98 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// Minimum of a 64-bit value over the wave (all lanes active).
-MK_DEV uint64_t wave_min_u64(uint64_t x) {
-  for (int off = 32; off >= 1; off >>= 1) {
-    const uint32_t lo = __shfl_xor(uint32_t(x), off, 64);
-    const uint32_t hi = __shfl_xor(uint32_t(x >> 32), off, 64);
-    const uint64_t o = (uint64_t(hi) << 32) | lo;
-    x = o < x ? o : x;
-  }
-  return x;
-}
-
-// Pull one in-chain of invalidated vertex tv (first slab word xv loaded):
-// the wave's minimum of dist[p] + w over valid, reached in-neighbours p is
-// applied to tv with one atomicMin.  Wave-collective.
+// Pull over one in-slab per 8-lane group (the group's invalidated vertex
+// tv, its lane's eight slab words w; `has`: the group has a slab): every
+// in-neighbour's invalid bit and distance are loaded together (with the
+// target's current value), the group's minimum of dist[p] + w over valid,
+// reached in-neighbours p is applied to tv with one atomicMin where it is
+// lower, and the improved vertices are pushed.  Where the wave's slabs are
+// one vertex's (a hub's buckets), they give one atomic: atomics on one
+// address serialise.  Wave-collective.
 template <bool MAP, bool WEIGHTS>
-MK_DEV void pull_chain(const GraphView &G, const GraphView &R, const TravView &S, WaveQ &q,
-                       uint32_t epoch, uint32_t tv, uint32_t xv, uint32_t &slabs,
-                       uint32_t &edges) {
-  const uint32_t lane = lane_id();
-  const bool key_lane = (key_mask<MAP>() >> lane) & 1ull;
-  for (;;) {
-    ++slabs;
-    const bool live = key_lane && xv < kTomb;
-    edges += uint32_t(__popcll(ballot(live)));
-    const uint32_t wv = MAP ? __shfl_down(xv, 1, 64) : 1u;
-    uint64_t cand = kInfInf;
-    if (live && !inv_bit(S.invbits, xv)) {
-      const uint32_t dp = dist_of(S.dist[xv]);
-      const uint32_t D = dp + (WEIGHTS ? wv : 1u);
-      if (dp != kInf && D >= dp) cand = pack(D, xv);
-    }
-    cand = wave_min_u64(cand);
-    bool push = false;
-    if (lane == 0 && cand != kInfInf) {
-      const uint64_t old = atomicMin((unsigned long long *)(S.dist + tv), (unsigned long long)cand);
-      if (dist_of(cand) < dist_of(old)) push = atomicExch(S.stamp + tv, epoch) != epoch;
-    }
-    enqueue(G, S, q, 0, 0, push, tv);
-    const uint32_t nx = read_lane(xv, kNextLane);
-    if (nx == kEmpty) break;
-    xv = slab_ptr(R.pool, nx)[lane];
-  }
-}
-
-// pull_chain over the head slabs of c <= kBatch in-buckets at once (slab k
-// of invalidated vertex tv[k], this lane's word x[k]), phase by phase so
-// that their dependent memory operations overlap: every in-neighbour's
-// invalid bit and distance are loaded together (with each target's
-// current value), the c wave minima are taken and merged per target, then
-// lane k applies slab k's minimum to tv[k] where it is lower (all atomics
-// in flight at once) and the improved vertices are pushed.  Chained slabs
-// follow one by one.  Wave-collective.
-template <bool MAP, bool WEIGHTS>
-MK_DEV void batch_pull_work(const GraphView &G, const GraphView &R, const TravView &S, WaveQ &q,
-                            uint32_t epoch, uint32_t c, const uint32_t (&tv)[kBatch],
-                            const uint32_t (&x)[kBatch], uint32_t &slabs, uint32_t &edges) {
-  const uint32_t lane = lane_id();
-  const bool key_lane = (key_mask<MAP>() >> lane) & 1ull;
-  // lane k < c: target tv[k] and its current value (a stale value only
-  // lets an extra atomic through: values only fall during the pull)
-  uint32_t t = 0;
+MK_DEV void group_pull_work(const GraphView &G, const TravView &S, WaveQ &q, uint32_t epoch,
+                            bool has, uint32_t tv, const uint32_t (&w)[kWordsPerLane],
+                            uint32_t &edges) {
+  constexpr uint32_t kStep = MAP ? 2 : 1, kKeys = kWordsPerLane / kStep;
+  const uint32_t gl = group_lane();
+  // a stale value only lets an extra atomic through: values only fall
+  // during the pull
+  const uint64_t tcur = has ? S.dist[tv] : 0ull;
+  bool live[kKeys];
+  uint32_t bits[kKeys];
+  uint64_t dp[kKeys];
 #pragma unroll
-  for (uint32_t k = 0; k < kBatch; ++k)
-    if (lane == k) t = tv[k];
-  const uint64_t tcur = lane < c ? S.dist[t] : 0ull;
-  bool live[kBatch];
-  uint32_t bits[kBatch], wv[kBatch];
-  uint64_t dp[kBatch];
-#pragma unroll
-  for (uint32_t k = 0; k < kBatch; ++k) {
-    live[k] = k < c && key_lane && x[k] < kTomb;
-    wv[k] = MAP ? __shfl_down(x[k], 1, 64) : 1u;
+  for (uint32_t k = 0; k < kKeys; ++k) {
+    const uint32_t x = w[k * kStep];
+    live[k] = has && key_word<MAP>(kWordsPerLane * gl + k * kStep) && x < kTomb;
     bits[k] = 0u;
     dp[k] = kInfInf;
     if (live[k]) {
-      bits[k] = S.invbits[x[k] >> 5];
-      dp[k] = S.dist[x[k]];
-    }
-  }
-  uint64_t cand[kBatch];
-#pragma unroll
-  for (uint32_t k = 0; k < kBatch; ++k) {
-    cand[k] = kInfInf;
-    if (live[k] && !((bits[k] >> (x[k] & 31u)) & 1u)) {
-      const uint32_t d = dist_of(dp[k]);
-      const uint32_t D = d + (WEIGHTS ? wv[k] : 1u);
-      if (d != kInf && D >= d) cand[k] = pack(D, x[k]);
+      bits[k] = S.invbits[x >> 5];
+      dp[k] = S.dist[x];
     }
     edges += uint32_t(__popcll(ballot(live[k])));
   }
+  uint64_t cand = kInfInf;
 #pragma unroll
-  for (uint32_t k = 0; k < kBatch; ++k) cand[k] = wave_min_u64(cand[k]);
-  // slabs of one vertex (a hub's buckets come in order) give one atomic:
-  // atomics on one address serialise
-#pragma unroll
-  for (uint32_t k = kBatch - 1; k > 0; --k)
-    if (k < c && tv[k - 1] == tv[k]) {
-      cand[k - 1] = cand[k] < cand[k - 1] ? cand[k] : cand[k - 1];
-      cand[k] = kInfInf;
+  for (uint32_t k = 0; k < kKeys; ++k) {
+    const uint32_t x = w[k * kStep];
+    if (live[k] && !((bits[k] >> (x & 31u)) & 1u)) {
+      const uint32_t d = dist_of(dp[k]);
+      const uint32_t D = d + (WEIGHTS ? w[k * kStep + (MAP ? 1 : 0)] : 1u);
+      if (d != kInf && D >= d) cand = min(cand, pack(D, x));
     }
-  uint64_t mine = kInfInf;
-#pragma unroll
-  for (uint32_t k = 0; k < kBatch; ++k)
-    if (lane == k) mine = cand[k];
+  }
+  const uint32_t t0 = first_lane_val(tv);
+  const bool one = ballot(has && tv == t0) == ~0ull;
+  for (uint32_t off = 1; off < (one ? 64u : kGroupLanes); off <<= 1) {
+    const uint32_t lo = uint32_t(__shfl_xor(int(uint32_t(cand)), int(off), 64));
+    const uint32_t hi = uint32_t(__shfl_xor(int(uint32_t(cand >> 32)), int(off), 64));
+    cand = min(cand, (uint64_t(hi) << 32) | lo);
+  }
   bool push = false;
-  if (mine < tcur) {
-    const uint64_t old = atomicMin((unsigned long long *)(S.dist + t), (unsigned long long)mine);
-    push = dist_of(mine) < dist_of(old);
+  if (has && (one ? lane_id() == 0 : gl == 0) && cand < tcur) {
+    const uint64_t old =
+        atomicMin((unsigned long long *)(S.dist + tv), (unsigned long long)cand);
+    push = dist_of(cand) < dist_of(old);
+    if (push) push = atomicExch(S.stamp + tv, epoch) != epoch;
   }
-  if (push) push = atomicExch(S.stamp + t, epoch) != epoch;
-  enqueue(G, S, q, 0, 0, push, t);
-  slabs += c;
-#pragma unroll
-  for (uint32_t k = 0; k < kBatch; ++k) {
-    const uint32_t nx = k < c ? read_lane(x[k], kNextLane) : kEmpty;
-    if (nx != kEmpty)
-      pull_chain<MAP, WEIGHTS>(G, R, S, q, epoch, tv[k], slab_ptr(R.pool, nx)[lane], slabs, edges);
-  }
+  enqueue(G, S, q, 0, 0, push, tv);
 }
 
 // Pull the in-buckets named by lanes of `m` (lane j: vertex tj, in-bucket
-// bk), kBatch head slabs at a time.
+// bk), eight at a time, one per 8-lane group, the next eight's slabs in
+// flight.
 template <bool MAP, bool WEIGHTS>
 MK_DEV void pull_buckets(const GraphView &G, const GraphView &R, const TravView &S, WaveQ &q,
                          uint32_t epoch, uint64_t m, uint32_t bk, uint32_t tj, uint32_t &slabs,
                          uint32_t &edges) {
-  const uint32_t lane = lane_id();
-  while (m) {
-    uint32_t js[kBatch];
-    uint32_t c = 0;
+  if (m == 0) return;
+  const uint32_t gl = group_lane(), grp = lane_id() / kGroupLanes;
+  const uint32_t n = uint32_t(__popcll(m));
+  const uint32_t from = pack_lanes(m);
+  const uint32_t bp = uint32_t(__shfl(int(bk), int(from), 64));
+  const uint32_t tp = uint32_t(__shfl(int(tj), int(from), 64));
+  uint32_t nxt[kWordsPerLane];
+  uint32_t bn = uint32_t(__shfl(int(bp), int(grp), 64));
+  if (grp < n) load_words(R.heads + size_t(bn) * kSlabWords + kWordsPerLane * gl, nxt);
+  for (uint32_t i = 0; i < n; i += kGroupsPerWave) {
+    uint32_t w[kWordsPerLane];
 #pragma unroll
-    for (uint32_t t = 0; t < kBatch; ++t) {
-      js[t] = m ? ffs64(m) : 0u;
-      if (m) {
-        m &= m - 1;
-        c = t + 1;
-      }
+    for (uint32_t k = 0; k < kWordsPerLane; ++k) w[k] = nxt[k];
+    bool has = i + grp < n;
+    const uint32_t t = uint32_t(__shfl(int(tp), int(i + grp), 64));
+    const uint32_t in = i + kGroupsPerWave + grp;
+    bn = uint32_t(__shfl(int(bp), int(in & 63u), 64));
+    if (in < n) load_words(R.heads + size_t(bn) * kSlabWords + kWordsPerLane * gl, nxt);
+    for (;;) {
+      slabs += uint32_t(__popcll(ballot(has && gl == 0)));
+      group_pull_work<MAP, WEIGHTS>(G, S, q, epoch, has, t, w, edges);
+      const uint32_t nx = group_read(w[kWordsPerLane - 1], kGroupLanes - 1);
+      has = has && nx != kEmpty;
+      if (ballot(has) == 0) break;
+      if (has) load_words(slab_ptr(R.pool, nx) + kWordsPerLane * gl, w);
     }
-    uint32_t x[kBatch], tv[kBatch];
-#pragma unroll
-    for (uint32_t t = 0; t < kBatch; ++t) {
-      x[t] = t < c ? R.heads[size_t(read_lane(bk, js[t])) * kSlabWords + lane] : kEmpty;
-      tv[t] = read_lane(tj, js[t]);
-    }
-    batch_pull_work<MAP, WEIGHTS>(G, R, S, q, epoch, c, tv, x, slabs, edges);
   }
 }
 
@@ -2588,7 +2535,7 @@ struct Traversal {
     // a BFS over a graph with the in-edge mirror may take bottom-up steps
     pull_now = persistent && vbits != nullptr;
     if (pull_now) fill_u32(vbits, 0u, uint64_t(bit_words()) * 2, stream);
-    bound_now = persistent && !pull_now && (weights || g->total_buckets > (1u << 19));
+    bound_now = persistent && !pull_now && g->total_buckets > (weights ? 1u << 17 : 1u << 19);
     if (bound_now) {
       fill_u32(reinterpret_cast<uint32_t *>(bound), ~0u, (uint64_t(g->n) + 1) / 2, stream);
       fill_u32(done, kInf, g->n, stream);
