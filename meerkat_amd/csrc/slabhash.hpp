@@ -212,6 +212,43 @@ MK_DEV uint32_t pool_alloc_group(const PoolView &P, uint32_t seed) {
   return kEmpty;
 }
 
+// Claim the free key word at `word` (holding `held`; a map: with the value
+// word behind it, one 64-bit swap writing key and value) for key dst.
+// Returns the key found: held's key if the claim succeeded (a free word's
+// value does not change during an insert kernel, so the keys tell).
+template <bool MAP>
+MK_DEV uint32_t claim_word(uint32_t *word, uint64_t held, uint32_t dst, uint32_t w) {
+  if (MAP)
+    return uint32_t(atomicCAS(reinterpret_cast<unsigned long long *>(word),
+                              (unsigned long long)held,
+                              ((unsigned long long)w << 32) | (unsigned long long)dst));
+  return atomicCAS(word, uint32_t(held), dst);
+}
+// The first free key word of the slab in `v` (load_slab_coherent's layout):
+// its index, with the words it holds in *held, or kSlabWords.  Group-wide.
+template <bool MAP>
+MK_DEV uint32_t first_free_word(const uint32_t (&v)[kWordsPerLane], uint64_t *held) {
+  const uint32_t gl = group_lane();
+  uint32_t fj = kWordsPerLane;  // this lane's first free key word
+#pragma unroll
+  for (int j = kWordsPerLane - 1; j >= 0; --j)
+    if (key_word<MAP>(coh_word(gl, j)) && v[j] >= kTomb) fj = uint32_t(j);
+  const uint32_t fb = group_bits(ballot(fj < kWordsPerLane));
+  if (!fb) return kSlabWords;
+  const uint32_t fl = ffs32(fb);
+  uint32_t key = 0, val = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < kWordsPerLane; ++j)
+    if (j == fj) {
+      key = v[j];
+      val = MAP && j + 1 < kWordsPerLane ? v[j + 1] : 0u;
+    }
+  key = group_read(key, fl);
+  val = MAP ? group_read(val, fl) : 0u;
+  *held = (uint64_t(val) << 32) | key;
+  return coh_word(fl, group_read(fj, fl));
+}
+
 // Insert (src -> dst [, w]) for one group (arguments group-uniform; `bucket` is
 // bucket_of(G, src, dst), computed by the caller for all its edges at once
 // so that this load leaves each operation's dependent chain).  `v` holds the
@@ -221,36 +258,39 @@ MK_DEV uint32_t pool_alloc_group(const PoolView &P, uint32_t seed) {
 // pointers from empty to a slab, so an older view can only show a taken
 // slot as free or a key as absent, and the claim made from it then fails
 // (the swap finds the slot taken) and the walk is redone from agent-scope
-// loads.  `v` is overwritten.  Returns 1 if inserted, 0 if already present,
-// -1 if the pool is exhausted.
+// loads.  `v` is overwritten; *head_view tells whether it ends as a view of
+// the bucket's only slab that shows the key.  Returns 1 if inserted, 0 if
+// already present, -1 if the pool is exhausted.
 template <bool MAP>
 MK_DEV int slab_insert_group(const GraphView &G, const PoolView &P, uint32_t bucket, uint32_t dst,
-                             uint32_t w, uint32_t seed, uint32_t (&v)[kWordsPerLane]) {
+                             uint32_t w, uint32_t seed, uint32_t (&v)[kWordsPerLane],
+                             bool *head_view) {
   const uint32_t gl = group_lane();
-  uint32_t *slab = G.heads + size_t(bucket) * kSlabWords;
+  uint32_t *const head = G.heads + size_t(bucket) * kSlabWords;
+  uint32_t *slab = head;
   uint32_t *free_slab = nullptr;
-  uint32_t free_word = 0, free_old = 0;
+  uint32_t free_word = 0;
+  uint64_t held = 0;
+  *head_view = false;
   for (;;) {
     bool hit = false;
-    uint32_t fj = kWordsPerLane;  // this lane's first free key word
 #pragma unroll
-    for (int j = kWordsPerLane - 1; j >= 0; --j) {
-      if (key_word<MAP>(coh_word(gl, j))) {
-        hit |= v[j] == dst;
-        if (v[j] >= kTomb) fj = uint32_t(j);
-      }
-    }
-    if (group_bits(ballot(hit))) return 0;
-    if (free_slab == nullptr) {
-      const uint32_t fb = group_bits(ballot(fj < kWordsPerLane));
-      if (fb) {
-        const uint32_t fl = ffs32(fb);
-        free_word = coh_word(fl, group_read(fj, fl));
-        free_old = group_read(fj < kWordsPerLane ? pick(v, fj) : 0u, fl);
-        free_slab = slab;
-      }
-    }
+    for (uint32_t j = 0; j < kWordsPerLane; ++j)
+      hit |= key_word<MAP>(coh_word(gl, j)) && v[j] == dst;
     const uint32_t nx = group_read(v[kWordsPerLane - 1], kGroupLanes - 1);  // word 63
+    if (group_bits(ballot(hit))) {
+      *head_view = slab == head && nx == kEmpty;
+      return 0;
+    }
+    if (free_slab == nullptr) {
+      uint64_t h = 0;
+      const uint32_t fw = first_free_word<MAP>(v, &h);
+      if (fw != kSlabWords) {
+        free_slab = slab;
+        free_word = fw;
+        held = h;
+      }
+    }
     if (nx != kEmpty) {
       slab = slab_ptr(G.pool, nx);
       load_slab_coherent(slab, v);
@@ -258,12 +298,19 @@ MK_DEV int slab_insert_group(const GraphView &G, const PoolView &P, uint32_t buc
     }
     if (free_slab != nullptr) {
       uint32_t old = 0;
-      if (gl == 0) {
-        old = atomicCAS(free_slab + free_word, free_old, dst);
-        if (MAP && old == free_old) free_slab[free_word + 1] = w;
-      }
+      if (gl == 0) old = claim_word<MAP>(free_slab + free_word, held, dst, w);
       old = group_read(old, 0);
-      if (old == free_old) return 1;
+      if (old == uint32_t(held)) {
+        // the claimed word in the view (word 16k + 2l + p is v[2k + p] of
+        // lane l): the bucket's next key of this group goes on from it
+        *head_view = slab == head;
+        const bool mine = gl == (free_word & 15u) >> 1;
+        const uint32_t fj = 2u * (free_word >> 4) + (free_word & 1u);
+#pragma unroll
+        for (uint32_t j = 0; j < kWordsPerLane; ++j)
+          if (mine && j == fj) v[j] = dst;
+        return 1;
+      }
       if (old == dst) return 0;
       slab = free_slab;  // lost the slot: re-walk from it
       free_slab = nullptr;
@@ -290,6 +337,38 @@ MK_DEV int slab_insert_group(const GraphView &G, const PoolView &P, uint32_t buc
     slab = slab_ptr(G.pool, old);
     load_slab_coherent(slab, v);
   }
+}
+
+// Where an insert of dst would go, given the bucket's head slab in `v`
+// (load_slab_coherent's layout; overwritten): 0 dst is present, 1 *slot is
+// the chain's first free word as walked (it held *held), 2 the chain is
+// full.  Nothing is claimed.  A claim of *slot made from it later keeps the
+// contract at the top of this file however old the walk is: it succeeds
+// only if the word is still free, and words never go from key to free
+// during an insert kernel.
+template <bool MAP>
+MK_DEV int slab_place_group(const GraphView &G, uint32_t bucket, uint32_t dst,
+                            uint32_t (&v)[kWordsPerLane], uint32_t **slot, uint64_t *held) {
+  const uint32_t gl = group_lane();
+  uint32_t *slab = G.heads + size_t(bucket) * kSlabWords;
+  uint32_t *at = nullptr;
+  for (;;) {
+    bool hit = false;
+#pragma unroll
+    for (uint32_t j = 0; j < kWordsPerLane; ++j)
+      hit |= key_word<MAP>(coh_word(gl, j)) && v[j] == dst;
+    if (group_bits(ballot(hit))) return 0;
+    if (at == nullptr) {
+      const uint32_t fw = first_free_word<MAP>(v, held);
+      if (fw != kSlabWords) at = slab + fw;
+    }
+    const uint32_t nx = group_read(v[kWordsPerLane - 1], kGroupLanes - 1);  // word 63
+    if (nx == kEmpty) break;
+    slab = slab_ptr(G.pool, nx);
+    load_slab_coherent(slab, v);
+  }
+  *slot = at;
+  return at ? 1 : 2;
 }
 
 // Delete (src -> dst) for one group: the key becomes a tombstone.  `v` holds the
