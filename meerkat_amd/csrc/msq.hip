@@ -38,7 +38,9 @@ constexpr uint32_t kMsSmall = 2;
 // and the counters of the one before (slot i-2).
 constexpr uint32_t kMsSlots = 4;
 
-struct MsCounts {
+constexpr uint32_t kMsStats = 16;
+
+struct alignas(64) MsCounts {
   uint32_t cnt[kMsSlots];          // small entries per slot
   uint32_t steps;                  // non-empty steps
   uint32_t pad0;
@@ -52,6 +54,13 @@ struct MsCounts {
   // bits the step writing it set, and of admissions into it); a source
   // missing from the queue of the next step has converged
   unsigned long long active[kMsSlots];
+  // SSSP: slots whose frontier is only its masks (no queue); per step, the
+  // buckets a scan expanded, and the totals, over kMsStats lines
+  uint32_t scan[kMsSlots];
+  struct alignas(64) Stat {
+    unsigned long long edges, slabs, pairs;
+    uint32_t width[kMsSlots];
+  } stat[kMsStats];
 };
 
 struct MsView {
@@ -327,18 +336,28 @@ __global__ void k_msbfs_read(MsView S, uint32_t s, uint32_t total, uint32_t leve
 }
 
 // ------------------------------------------------------------------ SSSP
-// Relax one slab of u for all sources in mu: per live key (neighbour v,
-// weight w), lanes are sources; four neighbours' distance rows are loaded at
-// a time.
 // A frontier vertex with at most this many active sources relaxes its slabs
 // key-parallel (lanes = neighbours, one pass per source) instead of
 // row-parallel (lanes = sources, neighbours a few at a time).
 constexpr uint32_t kMsSparse = 4;
+// Neighbours' distance rows a scan step keeps in flight per wave: 24 waves a
+// CU of them already draw all that memory gives for random 256-byte rows
+// (RMAT-20, 64 sources, a run's steps: 5.2 ms with 4 rows; 5.9 with 2, 5.4
+// with 3, 5.8 with 8, 7.6 with 16).
+constexpr uint32_t kMsScanRows = 4;
 
+// Relax one slab of u for all sources in mu: per live key (neighbour v,
+// weight w), lanes are sources; U neighbours' distance rows are loaded at a
+// time.  Neither the minimum nor (with `push` off) the mask update waits for
+// an old value: a candidate below the distance read marks its source bit
+// whether or not its own minimum lands last.  That sets no bit too many: a
+// distance read is never above the one the step began with, so some
+// candidate of this step improves it.  With `push`, a neighbour whose mask
+// was empty before is appended to the next queue.
 template <bool MAP, uint32_t U>
 MK_DEV void mssp_slab(const GraphView &G, const MsView &S, MsQ &q, uint32_t x, uint32_t du_lane,
-                      uint64_t mu, uint64_t *Fn, uint32_t *qn, uint32_t nslot, uint32_t &edges,
-                      uint64_t &pairs, uint64_t &acc) {
+                      uint64_t mu, uint64_t *Fn, uint32_t *qn, uint32_t nslot, bool push,
+                      uint32_t &edges, uint64_t &pairs, uint64_t &acc) {
   const uint32_t lane = lane_id();
   const uint64_t km = key_mask<MAP>();
   uint64_t live = ballot(x < kTomb) & km;
@@ -352,127 +371,160 @@ MK_DEV void mssp_slab(const GraphView &G, const MsView &S, MsQ &q, uint32_t x, u
       const uint32_t src = ffs64(m);
       const uint32_t du = read_lane(du_lane, src);
       if (du == kInf) continue;
-      bool push = false, imp = false;
+      bool fresh = false, imp = false;
       if (lv) {
         const uint32_t cand = du + wv;
         uint32_t *dp = S.dist + size_t(x) * 64 + src;
-        if (cand >= du && cand < *dp && cand < atomicMin(dp, cand)) {
-          imp = true;
-          push = atomicOr((unsigned long long *)(Fn + x), 1ull << src) == 0;
+        imp = cand >= du && cand < *dp;
+        if (imp) {
+          (void)atomicMin(dp, cand);
+          unsigned long long *fp = (unsigned long long *)(Fn + x);
+          if (push) fresh = atomicOr(fp, 1ull << src) == 0;
+          else (void)atomicOr(fp, 1ull << src);
         }
       }
       if (ballot(imp)) acc |= 1ull << src;
-      ms_push(G, S, q, push, x, qn, 0, &S.c->cnt[nslot], S.ql[nslot], &S.c->large[nslot], S.n,
-              false);
+      if (push)
+        ms_push(G, S, q, fresh, x, qn, 0, &S.c->cnt[nslot], S.ql[nslot], &S.c->large[nslot], S.n,
+                false);
     }
     return;
   }
-  const bool mine = (mu >> lane) & 1ull;
+  // only the lanes of sources active at u read their distance word, so a
+  // sparse mask touches one line of the 256-byte row, not both
+  const bool reads = ((mu >> lane) & 1ull) && du_lane != kInf;
+  uint64_t mine = 0;  // the sources improved at this lane's key
   while (live) {
-    uint32_t ks[U];
+    uint32_t ks[U], v[U], cur[U];
     uint32_t c = 0;
 #pragma unroll
     for (uint32_t qq = 0; qq < U; ++qq) {
-      ks[qq] = live ? ffs64(live) : 0u;
+      ks[qq] = v[qq] = 0u;
       if (live) {
+        ks[qq] = ffs64(live);
         live &= live - 1;
+        v[qq] = read_lane(x, ks[qq]);
         c = qq + 1;
       }
     }
-    // only the lanes of sources active at u read their distance word, so a
-    // sparse mask touches one line of the 256-byte row, not both
-    const bool reads = mine && du_lane != kInf;
-    uint32_t v[U], w[U], cur[U];
 #pragma unroll
-    for (uint32_t qq = 0; qq < U; ++qq) {
-      v[qq] = read_lane(x, ks[qq]);
-      w[qq] = MAP ? read_lane(x, ks[qq] + 1) : 1u;
-      cur[qq] = (qq < c && reads) ? S.dist[size_t(v[qq]) * 64 + lane] : 0u;
-    }
-    // the U neighbours' atomics are issued back to back (their round trips
-    // overlap), then the mask updates, then one push for all of them
-    uint32_t cand[U], old[U];
-    bool imp[U];
+    for (uint32_t qq = 0; qq < U; ++qq) cur[qq] = 0u;
+    if (reads) {
 #pragma unroll
-    for (uint32_t qq = 0; qq < U; ++qq) {
-      cand[qq] = du_lane + w[qq];
-      imp[qq] = qq < c && reads && cand[qq] >= du_lane && cand[qq] < cur[qq];
+      for (uint32_t qq = 0; qq < U; ++qq)
+        if (qq < c) cur[qq] = S.dist[size_t(v[qq]) * 64 + lane];
     }
 #pragma unroll
-    for (uint32_t qq = 0; qq < U; ++qq)
-      old[qq] = imp[qq] ? atomicMin(S.dist + size_t(v[qq]) * 64 + lane, cand[qq]) : 0u;
-    uint64_t im[U];
-#pragma unroll
     for (uint32_t qq = 0; qq < U; ++qq) {
-      im[qq] = ballot(imp[qq] && cand[qq] < old[qq]);
-      acc |= im[qq];
+      if (qq < c) {
+        // du + w < cur without overflow
+        const uint32_t w = MAP ? read_lane(x, ks[qq] + 1) : 1u;
+        const bool imp = w < __builtin_elementwise_sub_sat(cur[qq], du_lane);
+        const uint64_t im = ballot(imp);
+        if (im) {
+          if (imp) (void)atomicMin(S.dist + size_t(v[qq]) * 64 + lane, du_lane + w);
+          acc |= im;
+          if (lane == ks[qq]) mine = im;
+        }
+      }
     }
-    unsigned long long po[U];
-#pragma unroll
-    for (uint32_t qq = 0; qq < U; ++qq)
-      po[qq] = (im[qq] && lane == 0)
-                   ? atomicOr((unsigned long long *)(Fn + v[qq]), (unsigned long long)im[qq])
-                   : 1ull;
-    // neighbour qq is pushed (by lane qq) when its mask was empty before
-    uint32_t pm = 0;
-#pragma unroll
-    for (uint32_t qq = 0; qq < U; ++qq)
-      if (im[qq] && read_lane(uint32_t(po[qq] == 0), 0)) pm |= 1u << qq;
-    uint32_t vv = 0;
-#pragma unroll
-    for (uint32_t qq = 0; qq < U; ++qq)
-      if (lane == qq) vv = v[qq];
-    ms_push(G, S, q, lane < U && ((pm >> lane) & 1u), vv, qn, 0, &S.c->cnt[nslot], S.ql[nslot],
-            &S.c->large[nslot], S.n, false);
+  }
+  // one mask update for the slab: lane k its key's
+  if (ballot(mine != 0) == 0) return;
+  unsigned long long *fp = (unsigned long long *)(Fn + x);
+  if (push) {
+    bool fresh = false;
+    if (mine) fresh = atomicOr(fp, (unsigned long long)mine) == 0;
+    ms_push(G, S, q, fresh, x, qn, 0, &S.c->cnt[nslot], S.ql[nslot], &S.c->large[nslot], S.n,
+            false);
+  } else if (mine) {
+    (void)atomicOr(fp, (unsigned long long)mine);
   }
 }
 
 template <bool MAP, uint32_t U>
-MK_DEV void mssp_chain(const GraphView &G, const MsView &S, MsQ &q, uint32_t x, uint32_t u,
-                       uint64_t mu, uint64_t *Fn, uint32_t *qn, uint32_t nslot, uint32_t &edges,
-                       uint32_t &slabs, uint64_t &pairs, uint64_t &acc) {
-  const uint32_t du = S.dist[size_t(u) * 64 + lane_id()];
+MK_DEV void mssp_chain(const GraphView &G, const MsView &S, MsQ &q, uint32_t x, uint32_t du,
+                       uint64_t mu, uint64_t *Fn, uint32_t *qn, uint32_t nslot, bool push,
+                       uint32_t &edges, uint32_t &slabs, uint64_t &pairs, uint64_t &acc) {
   for (;;) {
     ++slabs;
-    mssp_slab<MAP, U>(G, S, q, x, du, mu, Fn, qn, nslot, edges, pairs, acc);
+    mssp_slab<MAP, U>(G, S, q, x, du, mu, Fn, qn, nslot, push, edges, pairs, acc);
     const uint32_t nx = read_lane(x, kNextLane);
     if (nx == kEmpty) break;
     x = slab_ptr(G.pool, nx)[lane_id()];
   }
 }
 
-// SSSP step i: queue slot i%4 (vertices, masks F[i%4]); appends to slot
-// (i+1)%4; clears the masks of queue i-1 (slot (i+3)%4) and the counters of
-// slot (i+2)%4 (queue i-2, whose masks step i-1 cleared).
-template <bool MAP, uint32_t U>
-__global__ void __launch_bounds__(kBlock) k_mssp_step(GraphView G, MsView S, uint32_t i) {
+// A step whose frontier has at least 1/kMsDense of the graph's buckets goes
+// over all buckets, looking up each one's mask, and leaves its next frontier
+// as masks alone: no queue, so no update waits for an old value (the queue
+// form waits for the minimum, the mask and the list position in turn).
+// RMAT-20, 64 sources: a step over all 16M edges 2.6 -> 1.0 ms, a run's steps
+// 13.4 -> 5.2 ms; bounded by the rows read past the L2 (3.2 GB a step).  The
+// least such frontier reads about what the scan's owner and mask words do.
+constexpr uint32_t kMsDense = 16;
+// Buckets a wave takes at a time (fewer even out the waves' work, and cost
+// owner and mask reads; 4, 6 and 8 were within 1% at RMAT-20, 4 the best by
+// 4-10% at RMAT-15 to 19).
+constexpr uint32_t kMsTake = 4;
+
+// The scan form of a step: every bucket whose vertex has sources in Fc.
+template <bool MAP>
+MK_DEV void mssp_scan(const GraphView &G, const MsView &S, MsQ &q, uint32_t gw, uint32_t W,
+                      const uint64_t *Fc, uint64_t *Fn, uint32_t *qn, uint32_t nslot, bool push,
+                      uint32_t &width, uint32_t &edges, uint32_t &slabs, uint64_t &pairs,
+                      uint64_t &acc) {
   const uint32_t lane = lane_id();
-  const uint32_t gw = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const uint32_t W = (gridDim.x * blockDim.x) >> 6;
-  const uint32_t slot = i % kMsSlots, nslot = (i + 1) % kMsSlots;
-  const uint32_t zslot = (i + 2) % kMsSlots, pslot = (i + 3) % kMsSlots;
-  const uint32_t count = S.c->cnt[slot];
-  const unsigned long long lg = S.c->large[slot];
-  const uint32_t n_large = uint32_t(lg >> 32);  // hub-list entries
-  uint32_t *qc = S.logv + size_t(slot) * S.n, *qn = S.logv + size_t(nslot) * S.n;
-  const uint32_t *qp = S.logv + size_t(pslot) * S.n;
-  uint64_t *Fc = S.F[slot], *Fn = S.F[nslot], *Fp = S.F[pslot];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    S.c->cnt[zslot] = 0;
-    S.c->large[zslot] = 0ull;
-    S.c->active[zslot] = 0ull;
+  const uint32_t T = G.total_buckets;
+  const uint32_t per = min(per_wave(T, W), kMsTake);
+  for (uint64_t k0 = uint64_t(gw) * per; k0 < T; k0 += uint64_t(W) * per) {
+    const uint64_t k = k0 + lane;
+    uint32_t u = 0;
+    uint64_t mu = 0;
+    if (lane < per && k < T) {
+      u = G.bucket_owner[k];
+      mu = Fc[u];
+    }
+    uint64_t m = ballot(mu != 0);
+    width += uint32_t(__popcll(m));
+    while (m) {
+      uint32_t js[4], x[4], du[4];
+      uint32_t c = 0;
+#pragma unroll
+      for (uint32_t qq = 0; qq < 4; ++qq) {
+        js[qq] = 0u;
+        x[qq] = kEmpty;
+        du[qq] = kInf;
+        if (m) {
+          js[qq] = ffs64(m);
+          m &= m - 1;
+          c = qq + 1;
+          x[qq] = G.heads[size_t(k0 + js[qq]) * kSlabWords + lane];
+          du[qq] = S.dist[size_t(read_lane(u, js[qq])) * 64 + lane];
+        }
+      }
+#pragma unroll 1
+      for (uint32_t qq = 0; qq < c; ++qq) {
+        const uint32_t xq = qq == 0 ? x[0] : qq == 1 ? x[1] : qq == 2 ? x[2] : x[3];
+        const uint32_t dq = qq == 0 ? du[0] : qq == 1 ? du[1] : qq == 2 ? du[2] : du[3];
+        const uint32_t jq = qq == 0 ? js[0] : qq == 1 ? js[1] : qq == 2 ? js[2] : js[3];
+        mssp_chain<MAP, kMsScanRows>(G, S, q, xq, dq, read_lane64(mu, jq), Fn, qn, nslot, push,
+                                     edges, slabs, pairs, acc);
+      }
+    }
   }
-  // queue i-1 is done: clear its masks before its slot is reused
-  const uint32_t pcount = i > 0 ? S.c->cnt[pslot] : 0u;
-  const uint32_t plarge = i > 0 ? uint32_t(S.c->large[pslot] >> 32) : 0u;
-  for (uint32_t k = gw * 64 + lane; k < pcount; k += W * 64) Fp[qp[k]] = 0ull;
-  for (uint32_t k = gw * 64 + lane; k < plarge; k += W * 64) Fp[S.ql[pslot][k].x] = 0ull;
-  if (count + n_large == 0) return;
-  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&S.c->steps, 1u);
-  __shared__ uint32_t lqbuf[kBlock / 64][kMsWaveQ];
-  MsQ q{lqbuf[threadIdx.x >> 6], 0u};
-  uint32_t edges = 0, slabs = 0;
-  uint64_t pairs = 0, acc = 0;  // acc: source bits improved into the next queue
+}
+
+// The queue form of a step: the hub list's buckets, then the small vertices.
+template <bool MAP, uint32_t U>
+MK_DEV void mssp_queue(const GraphView &G, const MsView &S, MsQ &q, uint32_t gw, uint32_t W,
+                       uint32_t slot, uint32_t nslot, uint32_t count, uint32_t n_large,
+                       uint32_t &edges, uint32_t &slabs, uint64_t &pairs, uint64_t &acc) {
+  const uint32_t lane = lane_id();
+  const uint32_t *qc = S.logv + size_t(slot) * S.n;
+  uint32_t *qn = S.logv + size_t(nslot) * S.n;
+  const uint64_t *Fc = S.F[slot];
+  uint64_t *Fn = S.F[nslot];
   const uint2 *ql = S.ql[slot];
   // lane l takes bucket l % kHubChunk of hub-list entry l / kHubChunk
   const uint32_t eper = min(per_wave(n_large, W), 64u / kHubChunk);
@@ -510,8 +562,9 @@ __global__ void __launch_bounds__(kBlock) k_mssp_step(GraphView G, MsView S, uin
       for (uint32_t qq = 0; qq < c; ++qq) {
         const uint32_t xq = qq == 0 ? x[0] : qq == 1 ? x[1] : qq == 2 ? x[2] : x[3];
         const uint32_t jq = qq == 0 ? js[0] : qq == 1 ? js[1] : qq == 2 ? js[2] : js[3];
-        mssp_chain<MAP, U>(G, S, q, xq, read_lane(u, jq), read_lane64(mu, jq), Fn, qn, nslot, edges,
-                           slabs, pairs, acc);
+        const uint32_t du = S.dist[size_t(read_lane(u, jq)) * 64 + lane];
+        mssp_chain<MAP, U>(G, S, q, xq, du, read_lane64(mu, jq), Fn, qn, nslot, true, edges, slabs,
+                           pairs, acc);
       }
     }
   }
@@ -534,17 +587,92 @@ __global__ void __launch_bounds__(kBlock) k_mssp_step(GraphView G, MsView S, uin
         const uint32_t j = ffs64(m);
         m &= m - 1;
         const uint32_t x = G.heads[size_t(read_lane(b0, j) + kk) * kSlabWords + lane];
-        mssp_chain<MAP, U>(G, S, q, x, read_lane(u, j), read_lane64(mu, j), Fn, qn, nslot, edges,
-                           slabs, pairs, acc);
+        const uint32_t du = S.dist[size_t(read_lane(u, j)) * 64 + lane];
+        mssp_chain<MAP, U>(G, S, q, x, du, read_lane64(mu, j), Fn, qn, nslot, true, edges, slabs,
+                           pairs, acc);
       }
     }
   }
+}
+
+// SSSP step i: the frontier of slot i%4 (masks F[i%4], and, unless scan[i%4],
+// its queue); leaves that of slot (i+1)%4; clears the masks of slot (i+3)%4
+// (step i-1's) and the counters of slot (i+2)%4 (queue i-2, whose masks step
+// i-1 cleared).
+template <bool MAP, uint32_t U>
+__global__ void __launch_bounds__(kBlock) k_mssp_step(GraphView G, MsView S, uint32_t i) {
+  const uint32_t lane = lane_id();
+  const uint32_t gw = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const uint32_t W = (gridDim.x * blockDim.x) >> 6;
+  const uint32_t slot = i % kMsSlots, nslot = (i + 1) % kMsSlots;
+  const uint32_t zslot = (i + 2) % kMsSlots, pslot = (i + 3) % kMsSlots;
+  const uint32_t count = S.c->cnt[slot];
+  const unsigned long long lg = S.c->large[slot];
+  const uint32_t n_large = uint32_t(lg >> 32);  // hub-list entries
+  uint32_t *qn = S.logv + size_t(nslot) * S.n;
+  const uint32_t *qp = S.logv + size_t(pslot) * S.n;
+  uint64_t *Fc = S.F[slot], *Fn = S.F[nslot], *Fp = S.F[pslot];
+  const bool masks = S.c->scan[slot] != 0;  // no queue was kept
+  const bool none = masks ? S.c->active[slot] == 0 : count + n_large == 0;
+  // buckets of this frontier (of one without a queue: as wide as the last)
+  uint64_t wide = uint64_t(count) + uint32_t(lg);
+  if (masks) {
+    const uint32_t wl = lane < kMsStats ? S.c->stat[lane].width[pslot] : 0u;
+    wide = wave_sum_u32(wl);
+  }
+  const bool dense = !none && wide * kMsDense >= G.total_buckets;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S.c->cnt[zslot] = 0;
+    S.c->large[zslot] = 0ull;
+    S.c->active[zslot] = 0ull;
+    S.c->scan[nslot] = dense ? 1u : 0u;
+  }
+  if (blockIdx.x == 0 && threadIdx.x < kMsStats) S.c->stat[threadIdx.x].width[zslot] = 0u;
+  // step i-1 is done: clear its masks before its slot is reused
+  if (i > 0 && S.c->scan[pslot]) {
+    for (uint32_t k = gw * 64 + lane; k < S.n; k += W * 64) Fp[k] = 0ull;
+  } else if (i > 0) {
+    const uint32_t pcount = S.c->cnt[pslot];
+    const uint32_t plarge = uint32_t(S.c->large[pslot] >> 32);
+    for (uint32_t k = gw * 64 + lane; k < pcount; k += W * 64) Fp[qp[k]] = 0ull;
+    for (uint32_t k = gw * 64 + lane; k < plarge; k += W * 64) Fp[S.ql[pslot][k].x] = 0ull;
+  }
+  if (none) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&S.c->steps, 1u);
+  __shared__ uint32_t lqbuf[kBlock / 64][kMsWaveQ];
+  MsQ q{lqbuf[threadIdx.x >> 6], 0u};
+  uint32_t edges = 0, slabs = 0;
+  uint64_t pairs = 0, acc = 0;  // acc: source bits improved into the next queue
+  uint32_t width = 0;
+  if (masks || dense) {
+    mssp_scan<MAP>(G, S, q, gw, W, Fc, Fn, qn, nslot, !dense, width, edges, slabs, pairs, acc);
+  } else {
+    mssp_queue<MAP, U>(G, S, q, gw, W, slot, nslot, count, n_large, edges, slabs, pairs, acc);
+  }
   ms_flush(S, q, qn, 0, &S.c->cnt[nslot], S.n);
-  acc = wave_or64(acc);  // wave-uniform already; the reduction keeps it exact
-  if (lane == 0 && acc) atomicOr(&S.c->active[nslot], (unsigned long long)acc);
-  if (lane == 0 && edges) atomicAdd(&S.c->edges, (unsigned long long)edges);
-  if (lane == 0 && slabs) atomicAdd(&S.c->slabs, (unsigned long long)slabs);
-  if (lane == 0 && pairs) atomicAdd(&S.c->pairs, (unsigned long long)pairs);
+  // totals: one add a block, spread over lines (adds to one line queue up)
+  __shared__ unsigned long long tot[3];
+  __shared__ uint32_t totw;
+  if (threadIdx.x < 3) tot[threadIdx.x] = 0ull;
+  if (threadIdx.x == 3) totw = 0u;
+  __syncthreads();
+  if (lane == 0 && slabs) {
+    atomicAdd(&tot[0], (unsigned long long)edges);
+    atomicAdd(&tot[1], (unsigned long long)slabs);
+    atomicAdd(&tot[2], (unsigned long long)pairs);
+    if (width) atomicAdd(&totw, width);
+  }
+  // (most waves find their bits set already)
+  if (lane == 0 && (acc & ~*(volatile unsigned long long *)&S.c->active[nslot]))
+    atomicOr(&S.c->active[nslot], (unsigned long long)acc);
+  __syncthreads();
+  MsCounts::Stat &st = S.c->stat[blockIdx.x % kMsStats];
+  if (threadIdx.x == 0 && tot[1]) {
+    atomicAdd(&st.edges, tot[0]);
+    atomicAdd(&st.slabs, tot[1]);
+    atomicAdd(&st.pairs, tot[2]);
+    if (totw) atomicAdd(&st.width[slot], totw);
+  }
 }
 
 __global__ void k_mssp_init(MsView S, const uint32_t *sources, uint32_t k) {
@@ -745,6 +873,11 @@ struct MultiSource {
     MK_HIP(hipMemcpyAsync(host.ptr, c, sizeof(MsCounts), hipMemcpyDeviceToHost, stream));
     MK_HIP(hipStreamSynchronize(stream));
     h = *host.as<MsCounts>();
+    for (const MsCounts::Stat &st : h.stat) {
+      h.edges += st.edges;
+      h.slabs += st.slabs;
+      h.pairs += st.pairs;
+    }
     return MK_OK;
   }
 
@@ -893,7 +1026,9 @@ struct MultiSource {
         MK_HIP(hipGetLastError());
         if (int r = read_counts(h)) return r;
         const uint32_t slot = step % (sssp ? kMsSlots : 3);
-        if (h.overflow || (h.cnt[slot] == 0 && (h.large[slot] >> 32) == 0)) break;
+        const bool drained = h.scan[slot] ? h.active[slot] == 0
+                                          : h.cnt[slot] == 0 && (h.large[slot] >> 32) == 0;
+        if (h.overflow || drained) break;
         if (step > limit || (!sssp && step + 1 >= g->n + 2))
           return fail(MK_ERR_STATE, "multi-source traversal did not drain");
         group = std::min<uint32_t>(group * 2, 8);
