@@ -47,19 +47,17 @@ struct alignas(64) MsCounts {
   unsigned long long large[kMsSlots];  // (hub-list entries << 32) | buckets per slot
   uint32_t overflow;               // log capacity exceeded
   uint32_t pad;
-  unsigned long long edges;        // adjacency entries read
-  unsigned long long slabs;        // slabs read
-  unsigned long long pairs;        // SSSP: (entry, active source) relaxations examined
   // per slot: the sources with an entry in that slot's queue (the OR of the
   // bits the step writing it set, and of admissions into it); a source
   // missing from the queue of the next step has converged
   unsigned long long active[kMsSlots];
-  // SSSP: slots whose frontier is only its masks (no queue); per step, the
-  // buckets a scan expanded, and the totals, over kMsStats lines
-  uint32_t scan[kMsSlots];
+  uint32_t scan[kMsSlots];  // SSSP: slots whose frontier is only its masks (no queue)
+  // totals over kMsStats lines
   struct alignas(64) Stat {
-    unsigned long long edges, slabs, pairs;
-    uint32_t width[kMsSlots];
+    unsigned long long edges;  // adjacency entries read
+    unsigned long long slabs;  // slabs read
+    unsigned long long pairs;  // SSSP: (entry, active source) relaxations examined
+    uint32_t width[kMsSlots];  // SSSP, per slot: the buckets a scan expanded
   } stat[kMsStats];
 };
 
@@ -132,6 +130,35 @@ MK_DEV void ms_push(const GraphView &G, const MsView &S, MsQ &q, bool push, uint
   if (to_list) q.buf[q.n + lanes_below(lm)] = v;
   q.n += c;
   push_hubs(G, ql, large, hub, v, nb);
+}
+
+// A step's totals: one add a block, spread over lines (adds to one line are
+// applied one after another, some 8 ns each: three a wave took 110 us of
+// every step).  `acc` is wave-uniform.  Block-collective, once per kernel.
+MK_DEV void add_totals(const MsView &S, uint32_t slot, uint32_t nslot, uint32_t edges,
+                       uint32_t slabs, uint64_t pairs, uint32_t width, uint64_t acc) {
+  __shared__ unsigned long long tot[3];
+  __shared__ uint32_t totw;
+  if (threadIdx.x < 3) tot[threadIdx.x] = 0ull;
+  if (threadIdx.x == 3) totw = 0u;
+  __syncthreads();
+  if (lane_id() == 0 && slabs) {
+    atomicAdd(&tot[0], (unsigned long long)edges);
+    atomicAdd(&tot[1], (unsigned long long)slabs);
+    atomicAdd(&tot[2], (unsigned long long)pairs);
+    if (width) atomicAdd(&totw, width);
+  }
+  // (most waves find their bits set already)
+  if (lane_id() == 0 && (acc & ~*(volatile unsigned long long *)&S.c->active[nslot]))
+    atomicOr(&S.c->active[nslot], (unsigned long long)acc);
+  __syncthreads();
+  MsCounts::Stat &st = S.c->stat[blockIdx.x % kMsStats];
+  if (threadIdx.x == 0 && tot[1]) {
+    atomicAdd(&st.edges, tot[0]);
+    atomicAdd(&st.slabs, tot[1]);
+    if (tot[2]) atomicAdd(&st.pairs, tot[2]);
+    if (totw) atomicAdd(&st.width[slot], totw);
+  }
 }
 
 // ------------------------------------------------------------------ BFS
@@ -288,25 +315,30 @@ __global__ void __launch_bounds__(kBlock) k_msbfs_level(GraphView G, MsView S, u
     }
   }
   ms_flush(S, q, S.logv, nbase, &S.c->cnt[nslot], S.log_cap);
-  acc = wave_or64(acc);
-  if (lane == 0 && acc) atomicOr(&S.c->active[nslot], (unsigned long long)acc);
-  if (lane == 0 && edges) atomicAdd(&S.c->edges, (unsigned long long)edges);
-  if (lane == 0 && slabs) atomicAdd(&S.c->slabs, (unsigned long long)slabs);
+  add_totals(S, slot, nslot, edges, slabs, 0, 0, wave_or64(acc));
 }
 
-__global__ void k_msbfs_init(MsView S, const uint32_t *sources, uint32_t k) {
-  // one thread: sources may repeat (same vertex in two slots)
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  uint32_t cntv = 0;
-  for (uint32_t s = 0; s < k; ++s) {
-    const uint32_t v = sources[s];
-    const uint64_t bit = 1ull << s;
-    if (S.F[0][v] == 0) S.logv[cntv++] = v;
-    S.F[0][v] |= bit;
-    S.seen[v] |= bit;
+// The first frontier, a lane per source (one wave; sources may repeat: the
+// same vertex in two slots).  64 sources, against one thread taking them in
+// turn: 41 -> 3 us.
+__global__ void __launch_bounds__(64) k_ms_init(MsView S, const uint32_t *sources, uint32_t k,
+                                                uint32_t sssp) {
+  const uint32_t s = threadIdx.x;
+  uint32_t v = 0;
+  bool fresh = false;
+  if (s < k) {
+    const unsigned long long bit = 1ull << s;
+    v = sources[s];
+    fresh = atomicOr((unsigned long long *)(S.F[0] + v), bit) == 0;
+    if (sssp) S.dist[size_t(v) * 64 + s] = 0;
+    else atomicOr((unsigned long long *)(S.seen + v), bit);
   }
-  S.seg[0] = 0;
-  S.c->cnt[0] = cntv;
+  const uint64_t m = ballot(fresh);
+  if (fresh) S.logv[lanes_below(m)] = v;
+  if (s == 0) {
+    if (!sssp) S.seg[0] = 0;
+    S.c->cnt[0] = uint32_t(__popcll(m));
+  }
 }
 
 // Hub vertices among the sources go to the hub list of slot 0 (one wave).
@@ -650,41 +682,7 @@ __global__ void __launch_bounds__(kBlock) k_mssp_step(GraphView G, MsView S, uin
     mssp_queue<MAP, U>(G, S, q, gw, W, slot, nslot, count, n_large, edges, slabs, pairs, acc);
   }
   ms_flush(S, q, qn, 0, &S.c->cnt[nslot], S.n);
-  // totals: one add a block, spread over lines (adds to one line queue up)
-  __shared__ unsigned long long tot[3];
-  __shared__ uint32_t totw;
-  if (threadIdx.x < 3) tot[threadIdx.x] = 0ull;
-  if (threadIdx.x == 3) totw = 0u;
-  __syncthreads();
-  if (lane == 0 && slabs) {
-    atomicAdd(&tot[0], (unsigned long long)edges);
-    atomicAdd(&tot[1], (unsigned long long)slabs);
-    atomicAdd(&tot[2], (unsigned long long)pairs);
-    if (width) atomicAdd(&totw, width);
-  }
-  // (most waves find their bits set already)
-  if (lane == 0 && (acc & ~*(volatile unsigned long long *)&S.c->active[nslot]))
-    atomicOr(&S.c->active[nslot], (unsigned long long)acc);
-  __syncthreads();
-  MsCounts::Stat &st = S.c->stat[blockIdx.x % kMsStats];
-  if (threadIdx.x == 0 && tot[1]) {
-    atomicAdd(&st.edges, tot[0]);
-    atomicAdd(&st.slabs, tot[1]);
-    atomicAdd(&st.pairs, tot[2]);
-    if (totw) atomicAdd(&st.width[slot], totw);
-  }
-}
-
-__global__ void k_mssp_init(MsView S, const uint32_t *sources, uint32_t k) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  uint32_t cntv = 0;
-  for (uint32_t s = 0; s < k; ++s) {
-    const uint32_t v = sources[s];
-    if (S.F[0][v] == 0) S.logv[cntv++] = v;
-    S.F[0][v] |= 1ull << s;
-    S.dist[size_t(v) * 64 + s] = 0;
-  }
-  S.c->cnt[0] = cntv;
+  add_totals(S, slot, nslot, edges, slabs, pairs, width, acc);
 }
 
 // Sources admitted into free slots of a running traversal (continuous
@@ -869,14 +867,15 @@ struct MultiSource {
     }
   }
 
+  // (the totals, summed, in h.stat[0])
   int read_counts(MsCounts &h) {
     MK_HIP(hipMemcpyAsync(host.ptr, c, sizeof(MsCounts), hipMemcpyDeviceToHost, stream));
     MK_HIP(hipStreamSynchronize(stream));
     h = *host.as<MsCounts>();
-    for (const MsCounts::Stat &st : h.stat) {
-      h.edges += st.edges;
-      h.slabs += st.slabs;
-      h.pairs += st.pairs;
+    for (uint32_t i = 1; i < kMsStats; ++i) {
+      h.stat[0].edges += h.stat[i].edges;
+      h.stat[0].slabs += h.stat[i].slabs;
+      h.stat[0].pairs += h.stat[i].pairs;
     }
     return MK_OK;
   }
@@ -994,7 +993,7 @@ struct MultiSource {
                                 "log four times larger)");
     }
     last_steps = h.steps;
-    last_edges = h.edges;
+    last_edges = h.stat[0].edges;
     *active = h.active[step % (sssp ? kMsSlots : 3)] & admitted;
     if (steps_done) *steps_done = step;
     return MK_OK;
@@ -1009,8 +1008,7 @@ struct MultiSource {
       MK_HIP(hipMemcpyAsync(src_dev, sources, nsrc * 4, hipMemcpyHostToDevice, stream));
       const GraphView G = g->view();
       const MsView S = view();
-      if (sssp) k_mssp_init<<<1, 64, 0, stream>>>(S, src_dev, nsrc);
-      else k_msbfs_init<<<1, 64, 0, stream>>>(S, src_dev, nsrc);
+      k_ms_init<<<1, 64, 0, stream>>>(S, src_dev, nsrc, sssp ? 1u : 0u);
       k_ms_source_hubs<<<1, 64, 0, stream>>>(G, S);
       MK_HIP(hipGetLastError());
       const unsigned grid = blocks_for_waves(uint64_t(max_waves));
@@ -1045,13 +1043,13 @@ struct MultiSource {
       if (ms) *ms = t;
       k = nsrc;
       last_steps = h.steps;
-      last_edges = h.edges;
+      last_edges = h.stat[0].edges;
       if (profiling_on())
         // BFS: 256 B per slab, 8 B per entry (the neighbour's seen mask);
         // SSSP: 256 B per slab, 4 B per (entry, active source) distance
         prof_add_bytes(sssp ? "k_mssp_step" : "k_msbfs_level",
-                       256.0 * double(h.slabs) +
-                           (sssp ? 4.0 * double(h.pairs) : 8.0 * double(h.edges)));
+                       256.0 * double(h.stat[0].slabs) +
+                           (sssp ? 4.0 * double(h.stat[0].pairs) : 8.0 * double(h.stat[0].edges)));
       if (!sssp) {
         // levels 0..steps-1 are non-empty; seg[steps] is the log length
         uint32_t segs[1];
