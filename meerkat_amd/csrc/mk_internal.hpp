@@ -129,18 +129,6 @@ MK_DEV uint32_t *slab_ptr(uint32_t *pool, uint32_t idx) {
   return pool + size_t(idx) * kSlabWords;
 }
 
-// Wave-aggregated append of the lanes with `pred` to queue[*count...].
-// Returns nothing; lanes with pred write their value.
-MK_DEV void wave_push(bool pred, uint32_t value, uint32_t *queue, uint32_t *count) {
-  uint64_t m = ballot(pred);
-  if (m == 0) return;
-  uint32_t base = 0;
-  uint32_t leader = ffs64(m);
-  if (lane_id() == leader) base = atomicAdd(count, uint32_t(__popcll(m)));
-  base = read_lane(base, leader);
-  if (pred) queue[base + lanes_below(m)] = value;
-}
-
 // Hub lists of the frontier kernels: an entry (vertex, global index of its
 // first bucket) per kHubChunk buckets of a listed vertex.
 constexpr uint32_t kHubChunk = 8;

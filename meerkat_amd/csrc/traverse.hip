@@ -11,8 +11,9 @@
 // Differences in method (same results):
 //  - The frontier holds vertices, not edges.  A wave takes up to 64 frontier
 //    vertices at once (their queue entries, bucket ranges and distances are
-//    read by all lanes in parallel) and then loads their bucket slabs four at
-//    a time, so several independent slab loads are in flight per wave.
+//    read by all lanes in parallel) and then works their bucket slabs in
+//    8-lane groups, eight at a time with the next eight loading (set slabs:
+//    those of hubs, and up to four of any, as one wave load each).
 //    Vertices with more than kSmallBuckets buckets are queued separately
 //    with a reserved range of "bucket work items" (one 64-bit atomicAdd
 //    returns the entry index and the range start together, so entries are
@@ -181,7 +182,6 @@ MK_DEV uint2 qload2(const uint2 *p) {
   const uint64_t x = coherent_load64(reinterpret_cast<const uint64_t *>(p));
   return make_uint2(uint32_t(x), uint32_t(x >> 32));
 }
-MK_DEV uint32_t qload2_y(const uint2 *p) { return qload(reinterpret_cast<const uint32_t *>(p) + 1); }
 
 MK_DEV void wq_flush(WaveQ &q, uint32_t *queue, uint32_t *count) {
   if (q.n == 0) return;
@@ -734,16 +734,10 @@ MK_DEV void batched_buckets(const GraphView &G, const TravView &S, Sink &sink, u
 }
 
 // Dense relax of the buckets named by lanes of `m` (as batched_buckets):
-// improved vertices get the step's epoch as their stamp (collect_step finds
-// them), by stores and atomics that nothing waits for, kDenseSlabs buckets
-// per 8-lane group at a time (their distance loads in flight together) and
-// the next ones' slabs on their way.
-MK_DEV void load_words_nt(const uint32_t *p, uint32_t (&v)[kWordsPerLane]) {
-  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-  const u4 *q = reinterpret_cast<const u4 *>(p);
-#pragma unroll
-  for (uint32_t k = 0; k < 2; ++k) { const u4 x = __builtin_nontemporal_load(q + k); v[4*k]=x.x; v[4*k+1]=x.y; v[4*k+2]=x.z; v[4*k+3]=x.w; }
-}
+// minima and bounds that nothing waits for (collect_step finds the improved
+// vertices), a slab per 8-lane group with the next one's words on their way.
+// Bounded by the gathers of the bounds; 2 or 3 slabs in flight per group
+// measured the same.
 template <bool MAP, bool WEIGHTS, bool HUB>
 MK_DEV void dense_buckets(const GraphView &G, const TravView &S, uint64_t m, uint32_t bk,
                           uint32_t uj, uint32_t dj, uint32_t &slabs, uint32_t &edges) {
