@@ -244,10 +244,11 @@ struct TravView {
   uint32_t delta;
   // Dense steps of a static run (bound == nullptr: other calls, none).
   // `bound`: upper bounds of the distances in 16 bits (kNoBound: none
-  // known), read in place of the 64-bit pairs: a quarter of their lines,
-  // most of which stay in L2.  Every improvement of the run stores its
-  // distance here; a bound that is out of date (stores that crossed, another
-  // XCD's copy) is only too high and lets an extra atomic through.
+  // known; kWide: a distance of kWide or more, which the pair tells), read
+  // in place of the 64-bit pairs: a quarter of their lines, most of which
+  // stay in L2.  Every improvement of the run stores its distance here; a
+  // bound that is out of date (stores that crossed, another XCD's copy) is
+  // only too high and lets an extra atomic through.
   // `done`: a distance at or above each one that the vertex's edges were all
   // relaxed with (kInf: none yet): a vertex whose distance has fallen below
   // it has to be expanded again.
@@ -259,12 +260,23 @@ struct TravView {
   const uint32_t *ep_base;
 };
 
-constexpr uint32_t kNoBound = 0xFFFFu;
+constexpr uint32_t kNoBound = 0xFFFFu, kWide = 0xFFFEu;
 // A static run improved v to d and, with `queued`, queues it for that.
 MK_DEV void note_improved(const TravView &S, uint32_t v, uint32_t d, bool queued) {
   if (!S.bound) return;
-  if (d < kNoBound) S.bound[v] = uint16_t(d);
+  S.bound[v] = uint16_t(min(d, kWide));
   if (queued) coherent_store(S.done + v, d);
+}
+// The distance that a candidate D for v has to be below, from v's bound:
+// kInf where none is known (so D = kInf, as unreached, is none).
+MK_DEV uint32_t dense_limit(const TravView &S, uint32_t v, uint32_t D, uint32_t bound) {
+  if (bound < kWide || (bound == kWide && D < kWide)) return bound;
+  return bound == kNoBound ? kInf : dist_of(S.dist[v]);
+}
+// Dense relax of v with D (below its limit `most`), from u.
+MK_DEV void dense_relax(const TravView &S, uint32_t v, uint32_t D, uint32_t u, uint32_t most) {
+  (void)atomicMin((unsigned long long *)(S.dist + v), (unsigned long long)pack(D, u));
+  if (D < kWide || most == kInf) S.bound[v] = uint16_t(min(D, kWide));
 }
 
 MK_DEV uint32_t wave_min_u32(uint32_t x) {
@@ -765,12 +777,11 @@ MK_DEV void dense_buckets(const GraphView &G, const TravView &S, uint64_t m, uin
         }
         more = false;
 #pragma unroll
+        for (uint32_t k = 0; k < kBatch; ++k)
+          if (most[k] >= kWide) most[k] = dense_limit(S, v[k], D[k], most[k]);
+#pragma unroll
         for (uint32_t k = 0; k < kBatch; ++k) {
-          if (D[k] != 0u && (D[k] < most[k] || most[k] == kNoBound)) {
-            (void)atomicMin((unsigned long long *)(S.dist + v[k]),
-                            (unsigned long long)pack(D[k], us[k]));
-            if (D[k] < kNoBound) S.bound[v[k]] = uint16_t(D[k]);
-          }
+          if (D[k] != 0u && D[k] < most[k]) dense_relax(S, v[k], D[k], us[k], most[k]);
           const uint32_t nx = read_lane(v[k], kNextLane);
           v[k] = nx != kEmpty ? slab_ptr(G.pool, nx)[lane] : kEmpty;
           slabs += nx != kEmpty ? 1u : 0u;
@@ -812,12 +823,13 @@ MK_DEV void dense_buckets(const GraphView &G, const TravView &S, uint64_t m, uin
       }
 #pragma unroll
       for (uint32_t k = 0; k < kKeys; ++k) {
-        const uint32_t v = w[k * kStep];
         const uint32_t D = du + (WEIGHTS ? w[k * kStep + (MAP ? 1 : 0)] : 1u);
-        if (D >= du && (D < most[k] || most[k] == kNoBound)) {
-          (void)atomicMin((unsigned long long *)(S.dist + v), (unsigned long long)pack(D, u));
-          if (D < kNoBound) S.bound[v] = uint16_t(D);
-        }
+        if (most[k] >= kWide) most[k] = dense_limit(S, w[k * kStep], D, most[k]);
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < kKeys; ++k) {
+        const uint32_t D = du + (WEIGHTS ? w[k * kStep + (MAP ? 1 : 0)] : 1u);
+        if (D >= du && D < most[k]) dense_relax(S, w[k * kStep], D, u, most[k]);
       }
       const uint32_t nx = group_read(w[kWordsPerLane - 1], kGroupLanes - 1);
       has = has && nx != kEmpty;
