@@ -785,8 +785,10 @@ struct PageRank {
     // heavy bins spread over the device.
     const uint64_t cap = std::max<uint64_t>(8192, m / plan.bins + m / plan.bins / 8);
     const uint64_t most = uint64_t(plan.bins) + m / cap + 1;
-    // an eighth to spare, so that growing graphs do not allocate at each call
-    if ((plan_words.bytes < m * 4 && plan_words.ensure((m + m / 8 + 64) * 4)) ||
+    // an eighth to spare, so that growing graphs do not allocate at each call;
+    // k_pr_iterate_bins reads four words at a time, the last ones included
+    const uint64_t word_bytes = (m + 3) / 4 * 16;
+    if ((plan_words.bytes < word_bytes && plan_words.ensure((m + m / 8 + 64) * 4)) ||
         (plan_items.bytes < most * 8 && plan_items.ensure((most + most / 8) * 8))) {
       (void)hipGetLastError();
       return false;

@@ -1,0 +1,36 @@
+"""PageRank over packed words whose number grows, call by call, to the end of
+the room kept to spare and past it, against the oracle's FP64 PageRank.
+
+Tolerance as for the other packed iterations: L1 <= 1e-6 against the ranks at
+delta 1e-14, for a stop at L1 delta 1e-7 (5.7e-7 of tail, 6e-8 of rounding).
+"""
+import numpy as np
+import pytest
+
+import meerkat_amd as mk
+import oracle
+from meerkat_amd import gen
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("first", [4001, 4002, 4007])
+def test_words_at_the_end_of_their_buffer(gpu, first):
+    n = 700
+    room = first + first // 8 + 64
+    s, d, _ = gen.insert_batch(None, n, room + 2, seed=first)
+    pool = mk.SlabPool(1 << 24)
+    g = mk.DynamicGraph(n, pool, 0.7, gen.degree_hints(n, s), reverse=True)
+    g.InsertEdges(s[:first], d[:first])
+    pr = mk.PageRank(g, 0.85, 1e-7)
+    pr.Static()
+    at = first
+    for upto in (room - 5, room - 3, room - 2, room - 1, room, room + 1, room + 2):
+        bs, bd = mk.device_u32(s[at:upto]), mk.device_u32(d[at:upto])
+        g.InsertEdges(bs, bd)
+        pr.Incremental(bs, bd)
+        at = upto
+        ref = oracle.csr(n, s[:at], d[:at])
+        want, _, delta = oracle.pagerank(oracle.transpose(ref), ref.degrees(), 0.85, 1e-14, 5000)
+        assert delta <= 1e-14 and pr.last_stats()["iterations"] > 2
+        assert np.abs(pr.Values().astype(np.float64) - want).sum() <= 1e-6
