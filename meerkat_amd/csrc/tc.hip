@@ -645,11 +645,17 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
+// Most work items at a time (32 MB): a batch that has more, hub-to-hub edges
+// mostly, is worked in passes over windows of them.
+constexpr uint64_t kMaxItems = 1ull << 22;
+
 // Work items of the changed edges: (edge, bucket of its enumerated end), the
-// edge's items side by side; one claim on *next per wave.
+// edge's items side by side; one claim on *next per wave.  With `start`
+// (batches of several windows) the claims, made by window 0, stay there, and
+// only the items lo, lo + 1, ... below hi are written.
 __global__ void __launch_bounds__(kBlock)
     k_tc_items(GraphView G, const uint2 *owned, uint32_t n_owned, uint2 *items,
-               unsigned long long *next) {
+               unsigned long long *next, unsigned long long *start, uint64_t lo, uint64_t hi) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t lane = lane_id();
   uint32_t nb = 0;
@@ -665,9 +671,17 @@ __global__ void __launch_bounds__(kBlock)
     if (lane >= o) incl += y;
   }
   unsigned long long base = 0;
-  if (lane == 63) base = atomicAdd(next, (unsigned long long)incl);
-  base = (uint64_t(read_lane(uint32_t(base >> 32), 63)) << 32) | read_lane(uint32_t(base), 63);
-  for (uint32_t j = 0; j < nb; ++j) items[base + incl - nb + j] = make_uint2(i, j);
+  if (lo == 0) {
+    if (lane == 63) base = atomicAdd(next, (unsigned long long)incl);
+    base = (uint64_t(read_lane(uint32_t(base >> 32), 63)) << 32) | read_lane(uint32_t(base), 63);
+    base += incl - nb;
+    if (start && nb) start[i] = base;
+  } else if (nb) {
+    base = start[i];
+  }
+  const uint32_t j0 = base < lo ? uint32_t(min<uint64_t>(lo - base, nb)) : 0u;
+  const uint32_t j1 = base < hi ? uint32_t(min<uint64_t>(hi - base, nb)) : 0u;
+  for (uint32_t j = j0; j < j1; ++j) items[base + j - lo] = make_uint2(i, j);
 }
 
 // Weight of a triangle with j changed edges: 6 / j.
@@ -845,7 +859,7 @@ struct TC {
   unsigned long long *slots = nullptr;
   uint32_t *n_owned = nullptr;  // [0] changed edges, [2..3] their items, [4..5] items written
   DevBuf tab, owned, ddeg, doff, cursor, dlist, scan_tmp, kup, koff, uplist, grabs;
-  DevBuf items;
+  DevBuf items, item_start;
   DevBuf ranks, rows, raw, slot, units;  // static count over sorted rows
   HostBuf host;
   unsigned long long count = 0;
@@ -873,7 +887,7 @@ struct TC {
     (void)hipFree(n_owned);
     for (DevBuf *b :
          {&tab, &owned, &ddeg, &doff, &cursor, &dlist, &scan_tmp, &kup, &koff, &uplist, &grabs,
-          &items, &ranks, &rows, &raw, &slot, &units})
+          &items, &item_start, &ranks, &rows, &raw, &slot, &units})
       b->release();
     host.release();
     if (ev0) (void)hipEventDestroy(ev0);
@@ -1086,7 +1100,8 @@ struct TC {
     return MK_OK;
   }
 
-  // Changed undirected edges of the batch into the set; returns their count.
+  // Changed undirected edges of the batch into the set, their count in m, that
+  // of their work items in nitems.
   int collect(const uint32_t *src, const uint32_t *dst, uint32_t n, int op, uint32_t &mask,
               uint32_t &m, uint64_t &nitems) {
     uint32_t cap = 1024;
@@ -1108,12 +1123,25 @@ struct TC {
     MK_HIP(hipStreamSynchronize(stream));
     m = host.as<uint32_t>()[0];
     nitems = host.as<uint64_t>()[1];
-    if (m) {
-      if (int r = items.ensure(nitems * 8)) return r;
-      k_tc_items<<<blocks_for_threads(m), kBlock, 0, stream>>>(
-          g->view(), owned.as<uint2>(), m, items.as<uint2>(), n_items + 1);
-    }
+    if (int r = items.ensure(std::min(nitems, kMaxItems) * 8)) return r;
+    if (nitems > kMaxItems)
+      if (int r = item_start.ensure(size_t(m) * 8)) return r;
     return MK_OK;
+  }
+
+  // Every work item of the m changed edges to `launch` (grid, items, their
+  // number), a window after the other.
+  template <typename F> void each_window(uint32_t m, uint64_t nitems, const F &launch) {
+    unsigned long long *written = reinterpret_cast<unsigned long long *>(n_owned + 4);
+    unsigned long long *start =
+        nitems > kMaxItems ? item_start.as<unsigned long long>() : nullptr;
+    for (uint64_t lo = 0; lo < nitems; lo += kMaxItems) {
+      const uint64_t hi = std::min(lo + kMaxItems, nitems);
+      k_tc_items<<<blocks_for_threads(m), kBlock, 0, stream>>>(
+          g->view(), owned.as<uint2>(), m, items.as<uint2>(), written, start, lo, hi);
+      launch(blocks_for_waves(std::min<uint64_t>(hi - lo, uint64_t(max_waves) * 2)),
+             items.as<uint2>(), hi - lo);
+    }
   }
 
   int run_incremental(const uint32_t *src, const uint32_t *dst, uint32_t n, float *ms) {
@@ -1125,12 +1153,13 @@ struct TC {
       uint64_t ni = 0;
       if (int r = collect(src, dst, n, 1, mask, m, ni)) return r;
       if (m) {
-        const unsigned grid = blocks_for_waves(std::min<uint64_t>(ni, uint64_t(max_waves) * 2));
         ProfScope prof(stream, "k_tc_inserted", 0.0);
         auto k = g->weighted ? k_tc_inserted<true> : k_tc_inserted<false>;
-        k<<<grid, kBlock, 0, stream>>>(g->view(), owned.as<uint2>(), items.as<uint2>(), ni,
-                                       tab.as<unsigned long long>(), mask, slots,
-                                       slots + kTcSlots);
+        each_window(m, ni, [&](unsigned grid, const uint2 *it, uint64_t count) {
+          k<<<grid, kBlock, 0, stream>>>(g->view(), owned.as<uint2>(), it, count,
+                                         tab.as<unsigned long long>(), mask, slots,
+                                         slots + kTcSlots);
+        });
       }
     }
     if (int r = finish(t, ms)) return r;
@@ -1167,12 +1196,14 @@ struct TC {
         k_tc_dfill<<<blocks_for_threads(m), kBlock, 0, stream>>>(
             owned.as<uint2>(), m, doff.as<uint32_t>(), cursor.as<uint32_t>(),
             dlist.as<uint32_t>());
-        const unsigned grid = blocks_for_waves(std::min<uint64_t>(ni, uint64_t(max_waves) * 2));
         ProfScope prof(stream, "k_tc_deleted", 0.0);
         auto k = g->weighted ? k_tc_deleted<true> : k_tc_deleted<false>;
-        k<<<grid, kBlock, 0, stream>>>(g->view(), owned.as<uint2>(), items.as<uint2>(), ni,
-                                       tab.as<unsigned long long>(), mask, doff.as<uint32_t>(),
-                                       dlist.as<uint32_t>(), slots, slots + kTcSlots);
+        each_window(m, ni, [&](unsigned grid, const uint2 *it, uint64_t count) {
+          k<<<grid, kBlock, 0, stream>>>(g->view(), owned.as<uint2>(), it, count,
+                                         tab.as<unsigned long long>(), mask,
+                                         doff.as<uint32_t>(), dlist.as<uint32_t>(), slots,
+                                         slots + kTcSlots);
+        });
       }
     }
     if (int r = finish(t, ms)) return r;
