@@ -464,8 +464,9 @@ int mk_msq_ready(mk_msq *q, int *ready);
  * without deferral); "sssp_far_cap" (default 0: one entry per vertex)
  * bounds each far list.  "tc_scratch_mb" (0..2^24, default 0: no bound,
  * read at each static count): most device scratch, in MB, of the static
- * triangle count's sorted lists (8 bytes per stored edge); a graph that
- * needs more is counted over plain lists (2 bytes per stored edge, slower).
+ * triangle count's sorted lists (8 bytes per stored edge, 48 per vertex and
+ * the degree sort's own); a graph that needs more is counted over plain lists
+ * (2 bytes per stored edge and 16 per vertex, slower).
  * The Python autotuner (meerkat_amd/autotune.py) sets them from
  * measurements. */
 int mk_tune_set(const char *name, int64_t value);

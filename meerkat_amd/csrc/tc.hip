@@ -922,13 +922,11 @@ struct TC {
     return MK_OK;
   }
 
-  // hipcub exclusive sum of n + 1 values on the handle's stream.
-  int exclusive_sum(const unsigned long long *in, unsigned long long *out) {
-    const int items = int(size_t(g->n) + 1);
-    size_t tmp = 0;
-    MK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, in, out, items, stream));
-    if (int r = scan_tmp.ensure(tmp)) return r;
-    MK_HIP(hipcub::DeviceScan::ExclusiveSum(scan_tmp.ptr, tmp, in, out, items, stream));
+  // hipcub exclusive sum of n + 1 values on the handle's stream, in scan_tmp
+  // (of `tmp` bytes at least).
+  int exclusive_sum(const unsigned long long *in, unsigned long long *out, size_t tmp) {
+    MK_HIP(hipcub::DeviceScan::ExclusiveSum(scan_tmp.ptr, tmp, in, out, int(size_t(g->n) + 1),
+                                            stream));
     return MK_OK;
   }
   int read_word(const unsigned long long *p, uint64_t &x) {
@@ -937,12 +935,30 @@ struct TC {
     x = *host.as<uint64_t>();
     return MK_OK;
   }
-  // Grow a buffer with an eighth to spare; false when memory is short.
-  static bool fits(DevBuf &b, uint64_t bytes) {
+  // The static count's scratch over sorted rows (uplist, scan_tmp and grabs
+  // are the plain lists' too).
+  uint64_t wedge_scratch() const {
+    uint64_t sum = 0;
+    for (const DevBuf *b : {&ranks, &rows, &raw, &slot, &units, &uplist, &scan_tmp, &grabs})
+      sum += b->bytes;
+    return sum;
+  }
+  // Grow a buffer of it, with an eighth to spare where nothing bounds it;
+  // false when memory is short, or past the bound (0: none).
+  bool fits(DevBuf &b, uint64_t bytes, uint64_t limit) {
     if (b.ptr && b.bytes >= bytes) return true;
-    if (b.ensure(bytes + bytes / 8) == MK_OK || b.ensure(bytes) == MK_OK) return true;
+    if (limit) {
+      if (wedge_scratch() - b.bytes + std::max<uint64_t>(bytes, 256) > limit) return false;
+    } else if (b.ensure(bytes + bytes / 8) == MK_OK) {
+      return true;
+    }
+    if (b.ensure(bytes) == MK_OK) return true;
     (void)hipGetLastError();
     return false;
+  }
+  void release_wedges() {
+    (void)hipStreamSynchronize(stream);
+    for (DevBuf *b : {&ranks, &rows, &raw, &slot, &units, &scan_tmp}) b->release();
   }
 
   // The wedge count queued on the stream (its result in `slots`), or
@@ -952,10 +968,14 @@ struct TC {
     *done = false;
     const uint32_t n = g->n;
     const uint64_t limit = uint64_t(tune_get("tc_scratch_mb", 0)) << 20;
+    if (limit && wedge_scratch() > limit) {  // grown without the bound
+      release_wedges();
+      uplist.release();
+    }
     // ranks: keys and values of the sort by (degree, id), both ways, and
     // the rank of each vertex; rows: places and lengths
     const size_t n1 = size_t(spread_rows(n)) * kSpread + 2;
-    if (!fits(ranks, n1 * 16) || !fits(rows, n1 * 32)) return MK_OK;
+    if (!fits(ranks, n1 * 16, limit) || !fits(rows, n1 * 32, limit)) return MK_OK;
     uint32_t *rank = ranks.as<uint32_t>(), *ids = rank + n1, *order = ids + n1, *sdeg = order + n1;
     unsigned long long *row0 = rows.as<unsigned long long>(), *off = row0 + n1, *tmp = off + n1;
     uint32_t *len = reinterpret_cast<uint32_t *>(tmp + n1), *ndown = len + n1;
@@ -966,19 +986,21 @@ struct TC {
     // degrees are below n (no self-loops, no duplicates)
     int bits = 1;
     while (bits < 32 && (n >> bits)) ++bits;
-    size_t need = 0;
+    size_t need = 0, scan = 0;
     MK_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, need, g->vdeg, sdeg, ids, order, int(n), 0,
                                               bits, stream));
-    if (!fits(scan_tmp, need)) return MK_OK;
+    MK_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, scan, tmp, row0, int(size_t(n) + 1), stream));
+    if (!fits(scan_tmp, std::max(need, scan), limit)) return MK_OK;
     MK_HIP(hipcub::DeviceRadixSort::SortPairs(scan_tmp.ptr, need, g->vdeg, sdeg, ids, order,
                                               int(n), 0, bits, stream));
     fill_u64(reinterpret_cast<uint64_t *>(tmp) + n, 0ull, 1, stream);
     k_tc_rank<<<tgrid, kBlock, 0, stream>>>(order, sdeg, n, rank, tmp);
-    if (int r = exclusive_sum(tmp, row0)) return r;
+    if (int r = exclusive_sum(tmp, row0, scan)) return r;
     uint64_t total = 0;
     if (int r = read_word(row0 + n, total)) return r;
-    if (limit && total * 8 > limit) return MK_OK;  // 4 B here and 4 B below a direction
-    if (!fits(raw, std::max<uint64_t>(total, 1) * 4)) return MK_OK;
+    // 4 B a direction here and 4 B below
+    if (limit && n1 * 48 + total * 8 > limit) return MK_OK;
+    if (!fits(raw, std::max<uint64_t>(total, 1) * 4, limit)) return MK_OK;
     fill_u32(len, 0u, 2 * n1, stream);  // and ndown
     const unsigned bgrid = blocks_for_waves(std::min<uint64_t>(
         (uint64_t(g->total_buckets) + 7) / 8, uint64_t(device_cus(g->device)) * 32));
@@ -986,26 +1008,27 @@ struct TC {
     kr<<<bgrid, kBlock, 0, stream>>>(g->view(), rank, row0, len, raw.as<uint32_t>(),
                                      slots + kTcSlots);
     k_tc_widen<<<blocks_for_threads(uint64_t(n) + 1), kBlock, 0, stream>>>(len, n, false, tmp);
-    if (int r = exclusive_sum(tmp, off)) return r;
+    if (int r = exclusive_sum(tmp, off, scan)) return r;
     uint64_t ups = 0;
     if (int r = read_word(off + n, ups)) return r;
     if (ups == 0) {
       *done = true;
       return MK_OK;
     }
-    if (!fits(uplist, ups * 4) || !fits(slot, ups * 4)) return MK_OK;
+    if (!fits(uplist, ups * 4, limit) || !fits(slot, ups * 4, limit)) return MK_OK;
     k_tc_sort<<<grid, kBlock, 0, stream>>>(row0, len, off, raw.as<uint32_t>(), n,
                                            uplist.as<uint32_t>(), slot.as<uint32_t>(), ndown);
     k_tc_widen<<<blocks_for_threads(uint64_t(n) + 1), kBlock, 0, stream>>>(ndown, n, true, tmp);
     unsigned long long *dof = row0;  // the raw rows' places are done with
-    if (int r = exclusive_sum(tmp, dof)) return r;
+    if (int r = exclusive_sum(tmp, dof, scan)) return r;
     uint64_t entries = 0;
     if (int r = read_word(dof + n, entries)) return r;
     const uint64_t nunits = (entries + kUnit - 1) / kUnit;
     // the lists take the raw rows' memory: two words an entry, at most one
     // entry per undirected edge of a graph that holds both directions
-    if (!fits(raw, std::max<uint64_t>(entries, 1) * 8) ||
-        !fits(units, std::max<uint64_t>(nunits, 1) * 4) || !fits(grabs, kTakers * 128))
+    if (!fits(raw, std::max<uint64_t>(entries, 1) * 8, limit) ||
+        !fits(units, std::max<uint64_t>(nunits, 1) * 4, limit) ||
+        !fits(grabs, kTakers * 128, limit))
       return MK_OK;
     if (entries) {
       unsigned long long *down = raw.as<unsigned long long>();
@@ -1042,6 +1065,7 @@ struct TC {
       count = t;
       return MK_OK;
     }
+    release_wedges();  // the plain lists may need their memory
     return run_static_lists(ms);
   }
 

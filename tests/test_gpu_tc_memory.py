@@ -1,11 +1,14 @@
 """Device memory of triangle counting: batches whose edges' buckets are more
-than the bound on work items (worked in windows, the count exact)."""
+than the bound on work items (worked in windows, the count exact), and
+the bound on the static count's scratch, which the fallback gives back."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import meerkat_amd as mk
-from meerkat_amd import gen
+from meerkat_amd import _lib, gen
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +52,40 @@ def test_batch_of_hub_edges(gpu, weighted, hubs, share):
         g.DeleteEdges(bi, bj)
         tc.Decremental(bi, bj)
         assert tc.GetCount() == 0
+
+
+@pytest.mark.parametrize("edges,mb", [(1000, 8), (4_000_000, 64)])
+def test_static_scratch_within_its_bound(gpu, edges, mb):
+    # 2^20 vertices: the sorted lists' per-vertex arrays (48 bytes) alone
+    # exceed 8 MB; with 8M directed entries they and the rows exceed 64 MB.
+    # The plain lists take 16 bytes a vertex and 4 an undirected edge.
+    n = 1 << 20
+    s, d, _ = gen.insert_batch(None, n // 2, edges, seed=edges)
+    keys = np.unique(np.r_[gen.keys_of(s, d), gen.keys_of(d, s)])
+    S, D = gen.split_keys(keys)
+    # and a clique of 60 on ids that the edges above do not touch
+    a, b = np.divmod(np.arange(3600, dtype=np.uint32), np.uint32(60))
+    m = a != b
+    A, B = a[m] + np.uint32(n - 60), b[m] + np.uint32(n - 60)
+    pool = mk.SlabPool(1 << 26)
+    g = mk.DynamicGraph(n, pool, 0.7, gen.degree_hints(n, np.r_[S, A]))
+    g.InsertEdges(np.r_[S, A], np.r_[D, B])
+    old = ctypes.c_int64()
+    _lib.call("mk_tune_get", b"tc_scratch_mb", ctypes.byref(old))
+    free, tc = mk.TC(g), mk.TC(g)
+    try:
+        _lib.call("mk_tune_set", b"tc_scratch_mb", 0)
+        free.Static()
+        want = free.GetCount()
+        assert want >= 60 * 59 * 58 // 6
+        _lib.call("mk_tune_set", b"tc_scratch_mb", mb)
+        for handle in (tc, free):  # a fresh one, and one that holds more
+            used = held(handle.Static)
+            assert handle.GetCount() == want
+            # plain lists 16 MB + 4 B an edge; four allocations rounded to 2 MB
+            assert used <= (24 << 20) + 4 * edges, used
+        _lib.call("mk_tune_set", b"tc_scratch_mb", 256)
+        assert held(tc.Static) <= 256 << 20
+        assert tc.GetCount() == want
+    finally:
+        _lib.call("mk_tune_set", b"tc_scratch_mb", old.value)
