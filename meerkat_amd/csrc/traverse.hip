@@ -1949,8 +1949,8 @@ struct Traversal {
   bool repair = false;  // orphan repair before invalidation (with the in-edge mirror)
   bool persistent = true;        // frontier steps in one launch (k_expand_loop)
   uint32_t tail_enter = 128;     // tail-mode entry threshold (knob "tail_enter")
-  uint16_t *bound = nullptr;     // 16-bit distance bounds (static runs)
-  uint32_t *done = nullptr;      // distances expanded with (static runs)
+  uint16_t *bound = nullptr;     // 16-bit distance bounds (static runs; null: no dense steps)
+  uint32_t *done = nullptr;      // distances expanded with (with `bound`)
   bool bound_now = false;        // the launch being queued is a static run's
   uint32_t *vbits = nullptr;     // two frontier bitmaps (static BFS with the mirror)
   uint32_t pull_enter = 0, pull_exit = 1;  // knobs "pull_enter" / "pull_exit"
@@ -2014,8 +2014,6 @@ struct Traversal {
     MK_HIP(hipMalloc(&stamp, n * 4));
     MK_HIP(hipMalloc(&invbits, ((n + 31) / 32) * 4));
     MK_HIP(hipMalloc(&inv_list, n * 4));
-    MK_HIP(hipMalloc(&bound, (n + 1) / 2 * 4));
-    MK_HIP(hipMalloc(&done, n * 4));
     for (int i = 0; i < 2; ++i) {
       MK_HIP(hipMalloc(&qs[i], n * 4));
       // one entry per kHubChunk buckets of every listed hub (a vertex is
@@ -2056,6 +2054,17 @@ struct Traversal {
     if (!weights && g->rev && pull_enter) {
       MK_HIP(hipMalloc(&vbits, size_t(bit_words()) * 8));
       if (int r = mirror_flags_enable(g->rev)) return r;
+    }
+    // dense steps: where a static run may take any (large frontiers, not
+    // bottom-up, not near-far) and there is memory for their arrays
+    if (persistent && !vbits && !far[0] && g->total_buckets > (weights ? 1u << 17 : 1u << 19)) {
+      if (hipMalloc(&bound, (n + 1) / 2 * 4) != hipSuccess ||
+          hipMalloc(&done, n * 4) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(bound);
+        bound = nullptr;
+        done = nullptr;
+      }
     }
     coop = tune_get("coop_launch", 0) != 0;
     loop_stream_add(g->device, stream, 1);
@@ -2546,7 +2555,7 @@ struct Traversal {
     // a BFS over a graph with the in-edge mirror may take bottom-up steps
     pull_now = persistent && vbits != nullptr;
     if (pull_now) fill_u32(vbits, 0u, uint64_t(bit_words()) * 2, stream);
-    bound_now = persistent && !pull_now && g->total_buckets > (weights ? 1u << 17 : 1u << 19);
+    bound_now = bound != nullptr;
     if (bound_now) {
       fill_u32(reinterpret_cast<uint32_t *>(bound), ~0u, (uint64_t(g->n) + 1) / 2, stream);
       fill_u32(done, kInf, g->n, stream);
