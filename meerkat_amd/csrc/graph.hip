@@ -440,15 +440,17 @@ MK_DEV MutSide pick_side(bool second, const MutSide &A, const MutSide &B) {
 // include/Graph/warp/InsertEdge.cuh:66-103).  Consecutive edges, which in a
 // batch sorted by source share buckets, so stay with one group, and the
 // groups in flight together work far-apart chunks instead of racing for
-// the same free slots.  A group whose edges all have different buckets
-// walks for each and then claims for all at once; otherwise it goes edge by
-// edge, keeping its view of a bucket from one edge to the next (reloading it
-// for each cost a lost claim and a re-walk an edge).  A map's key and value
-// are written by one 64-bit swap, a run of one source's edges adds its
-// degree once: swaps and degree adds (memory-side read-modify-writes of
-// random lines) are what bounds a random batch.  500k edges with the mirror
-// on RMAT-22: 139 -> 131 us; RMAT-20's 16.7M edges sorted by source, with
-// the mirror: 7.6 -> 4.0 ms.
+// the same free slots.  A group walks for each of its edges and then claims
+// for all at once; edges of one bucket, all in a batch sorted by source, then
+// claim the same word, and those that lose it go one by one (going edge by
+// edge throughout, the bucket's slab kept in registers from one to the next,
+// measured the same or up to 8% slower on sorted batches: 2.12 against
+// 2.02 ms for RMAT-20's 16.7M edges with weights, 1.68 against 1.48 without).
+// A map's key and value are written by one 64-bit swap, a run of one
+// source's edges adds its degree once: swaps and degree adds (memory-side
+// read-modify-writes of random lines) are what bounds a random batch.  500k
+// edges with the mirror on RMAT-22: 139 -> 131 us; RMAT-20's 16.7M edges
+// sorted by source, with weights and the mirror: 7.6 -> 3.9 ms.
 template <bool MAP>
 __global__ void __launch_bounds__(kBlock)
     k_insert(MutSide A, MutSide B, uint32_t waves_a, uint32_t waves_b, PoolView P,
@@ -498,67 +500,46 @@ __global__ void __launch_bounds__(kBlock)
   uint32_t pending = group_bits(ballot(act));
   uint32_t pool_fail = 0;
   const uint32_t seed_base = (second ? 0x9E3779B9u : 0u) + wave * 64u + group_first_lane();
-  // Two of the group's edges in one bucket?  (Never in a batch in random
-  // order, nearly always in one sorted by source.)
-  bool twin = false;
-#pragma unroll
-  for (uint32_t i = 0; i + 1 < kGroupLanes; ++i)
-    twin |= act && i < gl && ((pending >> i) & 1u) && group_read(bk, i) == bk;
-  const bool apart = group_bits(ballot(twin)) == 0u;
-  // head slabs with plain loads (an older view is safe: a claim made from it
-  // fails, and the walk is redone from agent-scope loads), the next edge's
-  // in flight while this one is worked
+  // every edge's walk first, then the lanes claim their edges' words
+  // together: one claim's round trip for all of them.  Head slabs with plain
+  // loads (an older view is safe: a claim made from it fails, and the walk is
+  // redone from agent-scope loads), the next edge's in flight meanwhile.
   uint32_t cur[kWordsPerLane], nxt[kWordsPerLane] = {};
-  bool done = false, retry = false;
   if (pending) load_slab_plain(G.heads + size_t(group_read(bk, ffs32(pending))) * kSlabWords, nxt);
-  if (apart) {
-    // every edge's walk first, then the lanes claim their edges' words
-    // together: one claim's round trip for all of them
-    uint32_t *slot = nullptr;
-    uint64_t held = 0;
-    int code = 0;  // slab_place_group of this lane's edge
-    for (uint32_t todo = pending; todo;) {
-      const uint32_t j = ffs32(todo);
-      todo &= todo - 1;
+  uint32_t *slot = nullptr;
+  uint64_t held = 0;
+  int code = 0;  // slab_place_group of this lane's edge
+  for (uint32_t todo = pending; todo;) {
+    const uint32_t j = ffs32(todo);
+    todo &= todo - 1;
 #pragma unroll
-      for (uint32_t k = 0; k < kWordsPerLane; ++k) cur[k] = nxt[k];
-      if (todo) load_slab_plain(G.heads + size_t(group_read(bk, ffs32(todo))) * kSlabWords, nxt);
-      uint32_t *sj = nullptr;
-      uint64_t hj = 0;
-      const int cj = slab_place_group<MAP>(G, group_read(bk, j), group_read(d, j), cur, &sj, &hj);
-      if (gl == j) {
-        slot = sj;
-        held = hj;
-        code = cj;
-      }
+    for (uint32_t k = 0; k < kWordsPerLane; ++k) cur[k] = nxt[k];
+    if (todo) load_slab_plain(G.heads + size_t(group_read(bk, ffs32(todo))) * kSlabWords, nxt);
+    uint32_t *sj = nullptr;
+    uint64_t hj = 0;
+    const int cj = slab_place_group<MAP>(G, group_read(bk, j), group_read(d, j), cur, &sj, &hj);
+    if (gl == j) {
+      slot = sj;
+      held = hj;
+      code = cj;
     }
-    retry = code == 2;
-    if (code == 1) {
-      const uint32_t old = claim_word<MAP>(slot, held, d, w);
-      done = old == uint32_t(held);
-      retry = !done && old != d;  // lost the word to another key
-    }
-    pending = group_bits(ballot(retry));  // one after another, from fresh loads
   }
-  bool view = false;  // cur shows the previous edge's bucket as it left it
-  uint32_t last = kEmpty;
+  bool done = false, retry = code == 2;
+  if (code == 1) {
+    const uint32_t old = claim_word<MAP>(slot, held, d, w);
+    done = old == uint32_t(held);
+    retry = !done && old != d;  // lost the word to another key
+  }
+  // those whose chain was full, or whose word another key took (another edge
+  // of the group, where several share a bucket), one after another
+  pending = group_bits(ballot(retry));
   while (pending) {
     const uint32_t j = ffs32(pending);
     pending &= pending - 1;
     const uint32_t bj = group_read(bk, j);
-    if (apart) {
-      load_slab_coherent(G.heads + size_t(bj) * kSlabWords, cur);
-    } else if (!(view && bj == last)) {
-#pragma unroll
-      for (uint32_t k = 0; k < kWordsPerLane; ++k) cur[k] = nxt[k];
-    }
-    // (for an edge of the same bucket, the view goes on: nothing to load)
-    if (!apart && pending && group_read(bk, ffs32(pending)) != bj) load_slab_plain(G.heads + size_t(group_read(bk, ffs32(pending))) * kSlabWords, nxt);
+    load_slab_coherent(G.heads + size_t(bj) * kSlabWords, cur);
     const int r = slab_insert_group<MAP>(G, P, bj, group_read(d, j), group_read(w, j),
-                                         seed_base + j, cur, &view);
-    last = bj;
-    if (!apart && !view && pending && group_read(bk, ffs32(pending)) == bj)
-      load_slab_coherent(G.heads + size_t(bj) * kSlabWords, nxt);
+                                         seed_base + j, cur);
     if (gl == j) done = r == 1;
     if (gl == j && r < 0) st = MK_EDGE_POOL_FULL;  // rolled back by the host
     if (r < 0) ++pool_fail;

@@ -258,30 +258,23 @@ MK_DEV uint32_t first_free_word(const uint32_t (&v)[kWordsPerLane], uint64_t *he
 // pointers from empty to a slab, so an older view can only show a taken
 // slot as free or a key as absent, and the claim made from it then fails
 // (the swap finds the slot taken) and the walk is redone from agent-scope
-// loads.  `v` is overwritten; *head_view tells whether it ends as a view of
-// the bucket's only slab that shows the key.  Returns 1 if inserted, 0 if
-// already present, -1 if the pool is exhausted.
+// loads.  `v` is overwritten.  Returns 1 if inserted, 0 if already present,
+// -1 if the pool is exhausted.
 template <bool MAP>
 MK_DEV int slab_insert_group(const GraphView &G, const PoolView &P, uint32_t bucket, uint32_t dst,
-                             uint32_t w, uint32_t seed, uint32_t (&v)[kWordsPerLane],
-                             bool *head_view) {
+                             uint32_t w, uint32_t seed, uint32_t (&v)[kWordsPerLane]) {
   const uint32_t gl = group_lane();
-  uint32_t *const head = G.heads + size_t(bucket) * kSlabWords;
-  uint32_t *slab = head;
+  uint32_t *slab = G.heads + size_t(bucket) * kSlabWords;
   uint32_t *free_slab = nullptr;
   uint32_t free_word = 0;
   uint64_t held = 0;
-  *head_view = false;
   for (;;) {
     bool hit = false;
 #pragma unroll
     for (uint32_t j = 0; j < kWordsPerLane; ++j)
       hit |= key_word<MAP>(coh_word(gl, j)) && v[j] == dst;
+    if (group_bits(ballot(hit))) return 0;
     const uint32_t nx = group_read(v[kWordsPerLane - 1], kGroupLanes - 1);  // word 63
-    if (group_bits(ballot(hit))) {
-      *head_view = slab == head && nx == kEmpty;
-      return 0;
-    }
     if (free_slab == nullptr) {
       uint64_t h = 0;
       const uint32_t fw = first_free_word<MAP>(v, &h);
@@ -300,17 +293,7 @@ MK_DEV int slab_insert_group(const GraphView &G, const PoolView &P, uint32_t buc
       uint32_t old = 0;
       if (gl == 0) old = claim_word<MAP>(free_slab + free_word, held, dst, w);
       old = group_read(old, 0);
-      if (old == uint32_t(held)) {
-        // the claimed word in the view (word 16k + 2l + p is v[2k + p] of
-        // lane l): the bucket's next key of this group goes on from it
-        *head_view = slab == head;
-        const bool mine = gl == (free_word & 15u) >> 1;
-        const uint32_t fj = 2u * (free_word >> 4) + (free_word & 1u);
-#pragma unroll
-        for (uint32_t j = 0; j < kWordsPerLane; ++j)
-          if (mine && j == fj) v[j] = dst;
-        return 1;
-      }
+      if (old == uint32_t(held)) return 1;
       if (old == dst) return 0;
       slab = free_slab;  // lost the slot: re-walk from it
       free_slab = nullptr;
