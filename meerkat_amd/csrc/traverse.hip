@@ -469,10 +469,11 @@ MK_DEV uint32_t wave_sum(uint32_t x) {
 
 MK_DEV bool inv_bit(const uint32_t *bits, uint32_t v) { return (bits[v >> 5] >> (v & 31u)) & 1u; }
 
-// Is D, the sum (mod 2^32) of a distance d and a weight, a distance?  Not
-// past 2^32, nor kInf itself, which stands for unreached: a re-seed storing
-// that sum would leave an unreached vertex with a parent.
-MK_DEV bool is_distance(uint32_t D, uint32_t d) { return D >= d && D != kInf; }
+// A re-seed's sum D of a distance d and a weight is a distance where D >= d
+// (not past 2^32) and D != kInf, which stands for unreached: storing that sum
+// would leave an unreached vertex with a parent.  (Relaxing compares D with a
+// distance anyway.)  Written out at its uses: as a function of D and d it had
+// the compiler spill 700 to 7400 scalar registers of the kernels over sets.
 
 // Per-slab work of the three passes.  `v` is this lane's word of one slab of
 // vertex u (distance du).  Wave-collective; returns live keys seen.
@@ -511,7 +512,7 @@ MK_DEV uint32_t slab_work(const GraphView &G, const TravView &S, Sink &sink, uin
   } else {  // re-seed invalidated v from valid u
     if (live && inv_bit(S.invbits, v)) {
       const uint32_t D = du + (WEIGHTS ? wv : 1u);
-      if (is_distance(D, du)) {
+      if (D >= du && D != kInf) {
         const uint64_t old = atomicMin((unsigned long long *)(S.dist + v),
                                        (unsigned long long)pack(D, u));
         if (D < dist_of(old)) push = atomicExch(S.stamp + v, epoch) != epoch;
@@ -553,7 +554,7 @@ MK_DEV uint32_t batch_slab_work(const GraphView &G, const TravView &S, Sink &sin
     live[k] = k < c && key_lane && v[k] < kTomb;
     const uint32_t wv = MAP ? __shfl_down(v[k], 1, 64) : 1u;
     D[k] = du[k] + (WEIGHTS ? wv : 1u);
-    ok[k] = live[k] && (MODE == 1 || is_distance(D[k], du[k]));
+    ok[k] = live[k] && (MODE == 1 || (D[k] >= du[k] && (!WEIGHTS || MODE != 2 || D[k] != kInf)));
     cur[k] = kInfInf;
     if (MODE == 2) {
       if (ok[k]) ok[k] = inv_bit(S.invbits, v[k]);
@@ -630,7 +631,7 @@ MK_DEV uint32_t group_slab_work(const GraphView &G, const TravView &S, Sink &sin
     const uint32_t v = w[k * kStep];
     live[k] = has && key_word<MAP>(kWordsPerLane * gl + k * kStep) && v < kTomb;
     D[k] = du + (WEIGHTS ? w[k * kStep + (MAP ? 1 : 0)] : 1u);
-    ok[k] = live[k] && (MODE == 1 || is_distance(D[k], du));
+    ok[k] = live[k] && (MODE == 1 || (D[k] >= du && (!WEIGHTS || MODE != 2 || D[k] != kInf)));
     cur[k] = kInfInf;
     if (MODE == 2) {
       if (ok[k]) ok[k] = inv_bit(S.invbits, v);
@@ -1476,7 +1477,7 @@ MK_DEV void group_pull_work(const GraphView &G, const TravView &S, WaveQ &q, uin
     if (live[k] && !((bits[k] >> (x & 31u)) & 1u)) {
       const uint32_t d = dist_of(dp[k]);
       const uint32_t D = d + (WEIGHTS ? w[k * kStep + (MAP ? 1 : 0)] : 1u);
-      if (d != kInf && is_distance(D, d)) cand = min(cand, pack(D, x));
+      if (d != kInf && D >= d && D != kInf) cand = min(cand, pack(D, x));
     }
   }
   const uint32_t t0 = first_lane_val(tv);
