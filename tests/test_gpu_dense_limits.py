@@ -38,8 +38,10 @@ def layers(k, ways, weights):
     (5, 0xFFFFFFFF - 5), (0xFFFFFFFE, 1), (0xFFFFFFF0, 0xF), (5, 0xFFFFFFFE - 5), (5, 0xFFFFFFFF),
 ])
 def test_sum_at_the_unreached_value(gpu, first, second):
-    # a frontier of 50,000 (past a dense step's least) of 150,001 buckets
-    n, s, d, w = layers(50_000, 1, [[first], [second], [7]])
+    # a frontier of 100,000 (past a dense step's least) of some 300,000
+    # buckets (past 2^18, so that the handle takes such steps)
+    k = 100_000
+    n, s, d, w = layers(k, 1, [[first], [second], [7]])
     g, ref = weighted_graph(n, s, d, w)
     sp = mk.SSSP(g, 0)
     for _ in range(2):
@@ -47,21 +49,21 @@ def test_sum_at_the_unreached_value(gpu, first, second):
         dist, par = sp.read()
         want = np.full(n, mk.INF, np.uint64)
         want[0] = 0
-        want[1:50_001] = first
+        want[1:k + 1] = first
         if first + second < mk.INF:
-            want[50_001:100_001] = first + second
+            want[k + 1:2 * k + 1] = first + second
             if first + second + 7 < mk.INF:
-                want[100_001:] = first + second + 7
+                want[2 * k + 1:] = first + second + 7
         assert np.array_equal(dist, want.astype(np.uint32))
         assert (par[dist == mk.INF] == mk.INF).all()
-        at = np.flatnonzero((dist != mk.INF) & (np.arange(n) > 50_000))
-        assert (par[at] == at - 50_000).all()
+        at = np.flatnonzero((dist != mk.INF) & (np.arange(n) > k))
+        assert (par[at] == at - k).all()
 
 
 @pytest.mark.parametrize("base", [65_533, 65_534, 65_535, 65_536, 1 << 20])
 def test_bounds_past_16_bits(gpu, base):
     # four offers a vertex, each step's later ones better or worse by one
-    n, s, d, w = layers(40_000, 4, [[base - 3], [3, 2, 1, 0], [0, 1, 2, 3], [1, 0, 1, 0],
+    n, s, d, w = layers(60_000, 4, [[base - 3], [3, 2, 1, 0], [0, 1, 2, 3], [1, 0, 1, 0],
                                     [70_000, 69_999, 1, 70_001]])
     g, ref = weighted_graph(n, s, d, w)
     sp = mk.SSSP(g, 0)
