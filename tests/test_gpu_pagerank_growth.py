@@ -9,7 +9,7 @@ import pytest
 
 import meerkat_amd as mk
 import oracle
-from meerkat_amd import gen
+from meerkat_amd import gen, profiling
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +34,26 @@ def test_words_at_the_end_of_their_buffer(gpu, first):
         want, _, delta = oracle.pagerank(oracle.transpose(ref), ref.degrees(), 0.85, 1e-14, 5000)
         assert delta <= 1e-14 and pr.last_stats()["iterations"] > 2
         assert np.abs(pr.Values().astype(np.float64) - want).sum() <= 1e-6
+
+
+def test_call_of_one_iteration_launches_one(gpu):
+    # ranks that still hold: the call ends with the wait after its first
+    # iteration
+    n, s, d, _ = gen.rmat(12, 8, seed=6)
+    pool = mk.SlabPool(1 << 26)
+    g = mk.DynamicGraph(n, pool, 0.7, gen.degree_hints(n, s), reverse=True)
+    g.InsertEdges(s, d)
+    pr = mk.PageRank(g, 0.85, 1e-6)
+    pr.Static()
+    many = pr.last_stats()["iterations"]
+    ranks = pr.Values()
+    profiling.enable()
+    try:
+        profiling.reset()
+        pr.Static()
+        used = profiling.totals()
+    finally:
+        profiling.enable(False)
+    assert many > 2 and pr.last_stats()["iterations"] == 1
+    assert used["k_pr_iterate"]["launches"] == 1
+    assert np.abs(pr.Values().astype(np.float64) - ranks).sum() <= 1e-6
