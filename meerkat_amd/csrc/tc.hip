@@ -256,6 +256,7 @@ constexpr uint32_t kTableWords = 1024;  // LDS words per wave: bitmap or hash ta
 constexpr uint32_t kTopRanks = kTableWords * 32;  // highest ranks a bitmap covers exactly
 constexpr uint32_t kUnit = 64;          // list entries per unit of k_tc_wedges
 constexpr uint32_t kTakers = 16;         // unit counters
+constexpr uint64_t kSmallTotal = 1u << 16;
 constexpr uint32_t kSortRow = 1024;     // row elements staged in LDS at a time
 constexpr uint32_t kTail = 8;           // lanes per tail
 constexpr uint32_t kRounds = 4;         // elements a lane takes at a time
@@ -539,6 +540,11 @@ __global__ void __launch_bounds__(kBlock)
                 const unsigned long long *doff, const unsigned long long *down,
                 const uint32_t *unit_b, uint32_t n, uint64_t entries, uint64_t units,
                 uint64_t stride, unsigned long long *next, unsigned long long *slots) {
+  if (entries == 0) {  // the host did not wait for them
+    entries = doff[n];
+    units = (entries + kUnit - 1) / kUnit;
+    stride = 1;
+  }
   __shared__ uint32_t table[kBlock / 64][kTableWords];
   uint32_t *tab = table[threadIdx.x >> 6];
   const uint32_t lane = lane_id();
@@ -859,6 +865,7 @@ struct TC {
   unsigned long long *slots = nullptr;
   uint32_t *n_owned = nullptr;  // [0] changed edges, [2..3] their items, [4..5] items written
   DevBuf tab, owned, ddeg, doff, cursor, dlist, scan_tmp, kup, koff, uplist, grabs;
+  uint32_t word_seq = 0;        // of read_word
   DevBuf items, item_start;
   DevBuf ranks, rows, raw, slot, units;  // static count over sorted rows
   HostBuf host;
@@ -875,7 +882,7 @@ struct TC {
     MK_HIP(hipEventCreate(&ev1));
     MK_HIP(hipMalloc(&slots, (kTcSlots + 2) * 8));
     MK_HIP(hipMalloc(&n_owned, 32));
-    if (int r = host.ensure((kTcSlots + 3) * 8)) return r;
+    if (int r = host.ensure((kTcSlots + 4) * 8)) return r;
     max_waves = grid_waves(g->device);
     return MK_OK;
   }
@@ -929,10 +936,13 @@ struct TC {
                                             stream));
     return MK_OK;
   }
+  // (through a word behind finish()'s; a copy and a stream wait cost 8 us more)
   int read_word(const unsigned long long *p, uint64_t &x) {
-    MK_HIP(hipMemcpyAsync(host.ptr, p, 8, hipMemcpyDeviceToHost, stream));
-    MK_HIP(hipStreamSynchronize(stream));
-    x = *host.as<uint64_t>();
+    constexpr uint32_t at = (kTcSlots + 2) * 2;
+    publish_words(reinterpret_cast<const uint32_t *>(p), static_cast<uint32_t *>(host.dev) + at, 2,
+                  ++word_seq, stream);
+    if (int r = host_wait_word(host.as<uint32_t>() + at + 2, word_seq, stream)) return r;
+    x = host.as<volatile uint64_t>()[kTcSlots + 2];
     return MK_OK;
   }
   // The static count's scratch over sorted rows (uplist, scan_tmp and grabs
@@ -996,11 +1006,16 @@ struct TC {
     fill_u64(reinterpret_cast<uint64_t *>(tmp) + n, 0ull, 1, stream);
     k_tc_rank<<<tgrid, kBlock, 0, stream>>>(order, sdeg, n, rank, tmp);
     if (int r = exclusive_sum(tmp, row0, scan)) return r;
-    uint64_t total = 0;
-    if (int r = read_word(row0 + n, total)) return r;
+    // Up to kSmallTotal stored edges the arrays are made for the most there
+    // can be, and the host waits for no length but this one, for none where n
+    // alone tells: each wait is some 10 us of a call of 75.
+    uint64_t total = uint64_t(n) * (n - 1);
+    if (limit || total > kSmallTotal)
+      if (int r = read_word(row0 + n, total)) return r;
+    const bool small = !limit && total <= kSmallTotal;
     // 4 B a direction here and 4 B below
     if (limit && n1 * 48 + total * 8 > limit) return MK_OK;
-    if (!fits(raw, std::max<uint64_t>(total, 1) * 4, limit)) return MK_OK;
+    if (!fits(raw, std::max<uint64_t>(total, 1) * (small ? 8 : 4), limit)) return MK_OK;
     fill_u32(len, 0u, 2 * n1, stream);  // and ndown
     const unsigned bgrid = blocks_for_waves(std::min<uint64_t>(
         (uint64_t(g->total_buckets) + 7) / 8, uint64_t(device_cus(g->device)) * 32));
@@ -1009,8 +1024,9 @@ struct TC {
                                      slots + kTcSlots);
     k_tc_widen<<<blocks_for_threads(uint64_t(n) + 1), kBlock, 0, stream>>>(len, n, false, tmp);
     if (int r = exclusive_sum(tmp, off, scan)) return r;
-    uint64_t ups = 0;
-    if (int r = read_word(off + n, ups)) return r;
+    uint64_t ups = total;
+    if (!small)
+      if (int r = read_word(off + n, ups)) return r;
     if (ups == 0) {
       *done = true;
       return MK_OK;
@@ -1021,8 +1037,9 @@ struct TC {
     k_tc_widen<<<blocks_for_threads(uint64_t(n) + 1), kBlock, 0, stream>>>(ndown, n, true, tmp);
     unsigned long long *dof = row0;  // the raw rows' places are done with
     if (int r = exclusive_sum(tmp, dof, scan)) return r;
-    uint64_t entries = 0;
-    if (int r = read_word(dof + n, entries)) return r;
+    uint64_t entries = ups;
+    if (!small)
+      if (int r = read_word(dof + n, entries)) return r;
     const uint64_t nunits = (entries + kUnit - 1) / kUnit;
     // the lists take the raw rows' memory: two words an entry, at most one
     // entry per undirected edge of a graph that holds both directions
@@ -1046,7 +1063,8 @@ struct TC {
       const unsigned wgrid = blocks_for_waves(
           std::min<uint64_t>(nunits, uint64_t(device_cus(g->device)) * 32));
       k_tc_wedges<<<wgrid, kBlock, 0, stream>>>(len, off, uplist.as<uint32_t>(), dof, down,
-                                                units.as<uint32_t>(), n, entries, nunits, stride,
+                                                units.as<uint32_t>(), n, small ? 0 : entries,
+                                                nunits, stride,
                                                 grabs.as<unsigned long long>(), slots);
     }
     MK_HIP(hipGetLastError());
