@@ -75,27 +75,51 @@ MK_DEV void uf_union(uint32_t *parent, uint32_t a, uint32_t b) {
 
 // Sampling steps before the edge pass.  Whole static passes, against finds
 // for both ends of every edge: RMAT-21 1.79 -> 0.67 ms, RMAT-18 0.64 -> 0.10,
-// ER 1M x 16M 0.76 -> 0.63, ER 1M x 1M 0.98 -> 0.33, a path of 1M vertices
+// ER 1M x 16M 0.75 -> 0.52, ER 1M x 1M 0.57 -> 0.30, a path of 1M vertices
 // 0.90 -> 0.14, a grid of 1M 0.69 -> 0.15.
-constexpr uint32_t kSampleSteps = 3;
+constexpr uint32_t kSampleSteps = 4;
 constexpr uint32_t kHookBlock = 1024;
+// The last step runs where kManyApart of kAsked vertices, spread over the
+// graph, still have a sampled key of another label: sparse uniform graphs,
+// whose trees join step by step, not RMAT ones, whose hubs have joined nearly
+// all.  Where many edges are left to k_cc_edges their unions meet on few
+// roots: weighted ER 131k x 1M took 2.0 ms with two keys a step (0.16 without
+// sampling, 0.12 now), ER 131k x 262k 0.65 without the last step (0.19, 0.11).
+// Small graphs leave few edges in any case, and the launches are a fifth of
+// their call (RMAT-14: 40 us with, 34 without).
+constexpr uint32_t kAsked = 1u << 14;
+constexpr uint32_t kManyApart = kAsked / 64;
+constexpr uint32_t kFewVertices = 1u << 15;
 
 __global__ void k_cc_init(uint32_t *parent, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) parent[i] = i;
 }
 
-// Keys of vertex u in words `word`, +1, +16 and +17 of its first slab (a map:
-// two of them): with word 0 the first that inserts fill.  kEmpty: none.
+// Four keys of vertex u in one line of its first slab: words `word`, +1, +16
+// and +17, of a map +0, +2, +16 and +18.  Inserts fill words 0, (1,) 16,
+// (17,) 32, (33,) 48, (49,) first, then 2, ....  kEmpty: none.
 template <bool MAP> MK_DEV void first_keys(const GraphView &G, uint32_t u, uint32_t word,
                                            uint32_t (&k)[4]) {
   const uint32_t *slab = G.heads + size_t(G.bucket_off[u]) * kSlabWords + word;
-  const uint2 a = *reinterpret_cast<const uint2 *>(slab);
-  const uint2 b = *reinterpret_cast<const uint2 *>(slab + 16);
-  k[0] = a.x < kTomb ? a.x : kEmpty;
-  k[1] = !MAP && a.y < kTomb ? a.y : kEmpty;
-  k[2] = b.x < kTomb ? b.x : kEmpty;
-  k[3] = !MAP && b.y < kTomb ? b.y : kEmpty;
+  if (MAP) {
+    const uint4 a = *reinterpret_cast<const uint4 *>(slab);
+    const uint4 b = *reinterpret_cast<const uint4 *>(slab + 16);
+    k[0] = a.x;
+    k[1] = a.z;
+    k[2] = b.x;
+    k[3] = b.z;
+  } else {
+    const uint2 a = *reinterpret_cast<const uint2 *>(slab);
+    const uint2 b = *reinterpret_cast<const uint2 *>(slab + 16);
+    k[0] = a.x;
+    k[1] = a.y;
+    k[2] = b.x;
+    k[3] = b.y;
+  }
+#pragma unroll
+  for (uint32_t q = 0; q < 4; ++q)
+    if (k[q] >= kTomb) k[q] = kEmpty;
 }
 
 // Sampling step 0: every vertex hangs under the smallest of itself and its
@@ -103,9 +127,11 @@ template <bool MAP> MK_DEV void first_keys(const GraphView &G, uint32_t u, uint3
 // vertices are followed in LDS right away, so that neighbours in id order
 // (paths, grids) make no long chains for the compress pass.
 template <bool MAP>
-__global__ void __launch_bounds__(kHookBlock) k_cc_hook(GraphView G, uint32_t *parent) {
+__global__ void __launch_bounds__(kHookBlock)
+    k_cc_hook(GraphView G, uint32_t *parent, uint32_t *apart) {
   __shared__ uint32_t lp[kHookBlock];
   const uint32_t t = threadIdx.x, base = blockIdx.x * kHookBlock, u = base + t;
+  if (u == 0) *apart = 0u;
   uint32_t p = u;
   if (u < G.n && G.vdeg[u] != 0) {
     uint32_t k[4];
@@ -127,19 +153,65 @@ __global__ void __launch_bounds__(kHookBlock) k_cc_hook(GraphView G, uint32_t *p
 // is smaller.  Of several offers to one root the smallest stays; the edges
 // of the others join in a later step or in k_cc_edges.  No step waits or
 // retries: finds and CAS loops from every vertex at once made chains that
-// took 0.3 ms on RMAT-21 and 8 ms on a path of 1M vertices.
+// took 0.3 ms on RMAT-21 and 8 ms on a path of 1M vertices.  With `apart`
+// (k_cc_ask's count), nothing unless there are many.
 template <bool MAP>
-__global__ void k_cc_sample(GraphView G, uint32_t *parent, uint32_t word) {
+__global__ void k_cc_sample(GraphView G, uint32_t *parent, uint32_t word,
+                            const uint32_t *apart) {
+  if (apart && *apart < kManyApart) return;
   const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= G.n || G.vdeg[u] == 0) return;
-  uint32_t k[4];
-  first_keys<MAP>(G, u, word, k);
-  const uint32_t pu = parent[u];
-  uint32_t lo = pu;
+  uint32_t pu = 0, lo = 0;
+  if (u < G.n && G.vdeg[u] != 0) {
+    uint32_t k[4];
+    first_keys<MAP>(G, u, word, k);
+    lo = pu = parent[u];
 #pragma unroll
-  for (uint32_t q = 0; q < 4; ++q)
-    if (k[q] != kEmpty) lo = min(lo, parent[k[q]]);
-  if (lo < pu && coherent_load(parent + pu) > lo) atomicMin(parent + pu, lo);
+    for (uint32_t q = 0; q < 4; ++q)
+      if (k[q] != kEmpty) lo = min(lo, parent[k[q]]);
+  }
+  bool offer = lo < pu;
+  uint64_t m = ballot(offer);
+  // two labels' offers go out once a wave: a large tree's vertices all have
+  // one for it, and accesses to one line follow one another (ER 131k x 1M,
+  // sorted: 0.40 -> 0.13 ms)
+  for (uint32_t t = 0; t < 2 && m; ++t) {
+    const uint32_t j = ffs64(m), label = read_lane(pu, j);
+    const bool same = offer && pu == label;
+    uint32_t best = same ? lo : kEmpty;
+#pragma unroll
+    for (uint32_t o = 32; o >= 1; o >>= 1)
+      best = min(best, uint32_t(__shfl_xor(int(best), int(o), 64)));
+    if (lane_id() == j && coherent_load(parent + label) > best) atomicMin(parent + label, best);
+    offer = offer && !same;
+    m = ballot(offer);
+  }
+  if (offer && coherent_load(parent + pu) > lo) atomicMin(parent + pu, lo);
+}
+
+// Of kAsked vertices, those with a sampled key of another label.
+template <bool MAP>
+__global__ void k_cc_ask(GraphView G, const uint32_t *parent, uint32_t *apart) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t u = uint32_t(uint64_t(i) * G.n / kAsked);
+  bool differs = false;
+  if (i < kAsked && G.vdeg[u] != 0) {
+    uint32_t k[4];
+    first_keys<MAP>(G, u, 0, k);
+    const uint32_t pu = parent[u];
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q)
+      if (k[q] != kEmpty) differs |= parent[k[q]] != pu;
+  }
+  const uint64_t m = ballot(differs);
+  if (m && lane_id() == 0) atomicAdd(apart, uint32_t(__popcll(m)));
+}
+
+// Union over edge (u, x) whose ends had labels pu and px: nothing where one
+// step up from the labels shows one component (a label that has been hung
+// under another one leaves a difference to all its edges).
+MK_DEV void join_labels(uint32_t *parent, uint32_t u, uint32_t x, uint32_t pu, uint32_t px) {
+  const uint32_t a = parent[pu], b = parent[px];
+  if (a != b && a != px && b != pu) uf_union(parent, u, x);
 }
 
 // Union over the edges whose ends have different labels: an 8-lane group per
@@ -166,7 +238,7 @@ __global__ void __launch_bounds__(kBlock) k_cc_edges(GraphView G, uint32_t *pare
         px[k] = key_word<MAP>(kWordsPerLane * gl + k) && x[k] < kTomb ? parent[x[k]] : pu;
 #pragma unroll
       for (uint32_t k = 0; k < kWordsPerLane; ++k)
-        if (px[k] != pu) uf_union(parent, u, x[k]);
+        if (px[k] != pu) join_labels(parent, u, x[k], pu, px[k]);
       const uint32_t nx = group_read(x[kWordsPerLane - 1], kGroupLanes - 1);
       if (nx == kEmpty) break;
       slab = slab_ptr(G.pool, nx);
@@ -196,7 +268,8 @@ __global__ void k_cc_compress(uint32_t *parent, uint32_t n) {
 // threads of a long chain shorten it together.  A halving store may land
 // after another thread's and leave an ancestor that is not the root: no
 // harm to the steps that follow, but labels end with k_cc_compress.
-__global__ void k_cc_shorten(uint32_t *parent, uint32_t n) {
+__global__ void k_cc_shorten(uint32_t *parent, uint32_t n, const uint32_t *apart) {
+  if (apart && *apart < kManyApart) return;
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) parent[i] = uf_find(parent, i);
 }
@@ -205,7 +278,7 @@ struct CC {
   mk_graph *g = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  uint32_t *parent = nullptr;
+  uint32_t *parent = nullptr;  // n parents (labels), then k_cc_ask's count
 
   int init(mk_graph *graph) {
     g = graph;
@@ -214,7 +287,7 @@ struct CC {
     loop_stream_add(g->device, stream, 1);
     MK_HIP(hipEventCreate(&ev0));
     MK_HIP(hipEventCreate(&ev1));
-    MK_HIP(hipMalloc(&parent, size_t(g->n) * 4));
+    MK_HIP(hipMalloc(&parent, (size_t(g->n) + 1) * 4));
     k_cc_init<<<blocks_for_threads(g->n), kBlock, 0, stream>>>(parent, g->n);
     MK_HIP(hipStreamSynchronize(stream));
     return MK_OK;
@@ -257,14 +330,19 @@ struct CC {
       ProfScope prof(stream, "k_cc_sample", kSampleSteps * 40.0 * g->n);
       auto hook = g->weighted ? k_cc_hook<true> : k_cc_hook<false>;
       auto sample = g->weighted ? k_cc_sample<true> : k_cc_sample<false>;
-      for (uint32_t step = 0; step < kSampleSteps; ++step) {
+      auto ask = g->weighted ? k_cc_ask<true> : k_cc_ask<false>;
+      uint32_t *apart = parent + g->n;
+      const uint32_t steps = g->n > kFewVertices ? kSampleSteps : kSampleSteps - 1;
+      for (uint32_t step = 0; step < steps; ++step) {
+        const uint32_t *when = step == kSampleSteps - 1 ? apart : nullptr;
+        if (when) ask<<<kAsked / kBlock, kBlock, 0, stream>>>(g->view(), parent, apart);
         if (step == 0)
           hook<<<unsigned((uint64_t(g->n) + kHookBlock - 1) / kHookBlock), kHookBlock, 0,
-                 stream>>>(g->view(), parent);
+                 stream>>>(g->view(), parent, apart);
         else
           sample<<<blocks_for_threads(g->n), kBlock, 0, stream>>>(g->view(), parent,
-                                                                  step == 1 ? 0 : 32);
-        k_cc_shorten<<<blocks_for_threads(g->n), kBlock, 0, stream>>>(parent, g->n);
+                                                                  step == 2 ? 32 : 0, when);
+        k_cc_shorten<<<blocks_for_threads(g->n), kBlock, 0, stream>>>(parent, g->n, when);
       }
     }
     {
