@@ -683,7 +683,11 @@ MK_DEV uint32_t group_slab_work(const GraphView &G, const TravView &S, Sink &sin
 // vertex uj with distance dj).  Eight buckets at a time, one per 8-lane
 // group, their head slabs loaded together and the next eight's in flight;
 // chained slabs follow, the groups that have one together (static SSSP on
-// RMAT-24: 17.3 ms with a slab a wave throughout, 14.2 in groups).  Set
+// RMAT-24: 17.3 ms with a slab a wave throughout, 14.2 in groups), the last
+// of them by the whole wave: a hub's chain in a graph without degree hints
+// is a serial walk, longer the more keys a lane has (RMAT-15, 32 edges a
+// vertex, SSSP: 3.9 ms to its end by a group, 2.7 so, 2.5 by waves
+// throughout; BFS over sets on RMAT-17, 2.3, 0.84 and 0.85 ms).  Set
 // slabs, eight key words a lane, are worked in groups only where a wave has
 // many nearly empty ones: a hub's (HUB) are full, a key for nearly every
 // lane (BFS on RMAT-16: its hub step 32 us so, 72 us in groups), and up to
@@ -745,7 +749,18 @@ MK_DEV void batched_buckets(const GraphView &G, const TravView &S, Sink &sink, u
       edges += group_slab_work<MAP, WEIGHTS, MODE>(G, S, sink, epoch, has, u, du, w);
       const uint32_t nx = group_read(w[kWordsPerLane - 1], kGroupLanes - 1);
       has = has && nx != kEmpty;
-      if (ballot(has) == 0) break;
+      uint64_t more = ballot(has);
+      if (more == 0) break;
+      // few chains left: one after another, a key a lane
+      if (__popcll(more) <= int(kGroupLanes * (MAP ? 1 : 2))) {
+        for (; more; more &= ~(uint64_t(kGroupMask) << (ffs64(more) & ~(kGroupLanes - 1)))) {
+          const uint32_t l = ffs64(more);
+          chain_work<MAP, WEIGHTS, MODE>(G, S, sink, epoch, read_lane(u, l), read_lane(du, l),
+                                         slab_ptr(G.pool, read_lane(nx, l))[lane_id()], slabs,
+                                         edges);
+        }
+        break;
+      }
       if (has) load_words(slab_ptr(G.pool, nx) + kWordsPerLane * gl, w);
     }
   }
