@@ -721,6 +721,13 @@ struct PageRank {
       // 2^12 a bin, 1.1 to 2 times slower two steps away.
       uint32_t bits = 8;
       while (bits < kBinMaxBits && (g->n >> (bits + 1)) >= 256) ++bits;
+      // Fewer vertices with many edges each: smaller bins, so that the
+      // device is full (some 20 keys a bucket of a map, 40 of a set).  A
+      // clique of 2000, 64 of 300: calls of several iterations 1.05 and 0.61
+      // ms with 8 and 75 bins, 0.50 and 0.56 with 63 and 300 (walks over the
+      // slabs 0.46 and 0.56).
+      const uint64_t keys = uint64_t(in->total_buckets) * (in->weighted ? 20 : 40);
+      while (bits > 5 && (g->n >> bits) < 256 && (keys >> 14) > (g->n >> bits)) --bits;
       PrPlan L{};
       L.bin_bits = bits;
       L.bins = uint32_t((uint64_t(g->n) + (1u << bits) - 1) >> bits);

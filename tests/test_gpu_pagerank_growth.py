@@ -57,3 +57,23 @@ def test_call_of_one_iteration_launches_one(gpu):
     assert many > 2 and pr.last_stats()["iterations"] == 1
     assert used["k_pr_iterate"]["launches"] == 1
     assert np.abs(pr.Values().astype(np.float64) - ranks).sum() <= 1e-6
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("n,degree", [(600, 500), (3001, 400), (16_385, 250), (9000, 700)])
+def test_small_bins(gpu, n, degree, weighted):
+    # many edges a vertex: bins of 32 to 128 vertices, the last not full
+    s, d, _ = gen.insert_batch(None, n, n * degree, seed=n)
+    hub = np.arange(1, n, dtype=np.uint32)  # one vertex that all others name
+    keys = np.unique(np.r_[gen.keys_of(s, d), gen.keys_of(hub, np.zeros(n - 1, np.uint32))])
+    s, d = gen.split_keys(keys)
+    pool = mk.SlabPool(1 << 28)
+    g = mk.DynamicGraph(n, pool, 0.7, gen.degree_hints(n, s), weighted=weighted, reverse=True,
+                        in_degree_hints=gen.degree_hints(n, d))
+    g.InsertEdges(s, d, np.ones(len(s), np.uint32) if weighted else None)
+    pr = mk.PageRank(g, 0.85, 1e-7)
+    pr.Static()
+    ref = oracle.csr(n, s, d)
+    want, _, delta = oracle.pagerank(oracle.transpose(ref), ref.degrees(), 0.85, 1e-14, 5000)
+    assert delta <= 1e-14 and pr.last_stats()["iterations"] > 2
+    assert np.abs(pr.Values().astype(np.float64) - want).sum() <= 1e-6
