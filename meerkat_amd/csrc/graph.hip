@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstring>
 #include <map>
 #include <numeric>
@@ -165,25 +166,32 @@ int host_wait_word(const volatile uint32_t *word, uint32_t want, hipStream_t s) 
 
 // ---------------------------------------------------------------- readback
 // The pinned slots of read_chunks: kReadSlots chunks, then a line of flag
-// words per slot and block group.  One reader at a time holds `mu`.
-static struct ReadStage {
+// words per slot and block group.  A reader holds `mu` of the stage it uses
+// while it waits for the work queued before its chunks; there are several,
+// allocated as reads overlap.  (Waiting for the stream first, to need only
+// one, took 20 to 30 us more a read: 10 -> 40 us for 64 words.)
+struct ReadStage {
   std::mutex mu;
   uint32_t *ptr = nullptr, *dev = nullptr;
   uint32_t seq = 0;  // of the last chunk
-  int pools = 0;     // slab pools alive: the stage is freed with the last
-} g_read;
+};
+static ReadStage g_read[kReadStages];
+static std::mutex g_read_pools_mu;
+static int g_read_pools = 0;  // slab pools alive: the stages are freed with the last
 
 static void read_stage_pool(int delta) {
-  std::lock_guard<std::mutex> lk(g_read.mu);
-  if ((g_read.pools += delta) <= 0 && g_read.ptr) {
-    (void)hipHostFree(g_read.ptr);
-    g_read.ptr = g_read.dev = nullptr;
+  std::lock_guard<std::mutex> pl(g_read_pools_mu);
+  if ((g_read_pools += delta) > 0) return;
+  for (ReadStage &st : g_read) {
+    std::lock_guard<std::mutex> lk(st.mu);
+    if (st.ptr) (void)hipHostFree(st.ptr);
+    st.ptr = st.dev = nullptr;
   }
 }
 
-// Caller holds g_read.mu.  False where pinned memory is short.
-static bool read_stage_ready() {
-  if (g_read.ptr) return true;
+// Caller holds st.mu.  False where pinned memory is short.
+static bool read_stage_ready(ReadStage &st) {
+  if (st.ptr) return true;
   const size_t words = size_t(kReadSlots) * (kReadWords + kReadBlocks);
   void *p = nullptr, *d = nullptr;
   if (hipHostMalloc(&p, words * 4, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
@@ -197,10 +205,22 @@ static bool read_stage_ready() {
   }
   std::memset(static_cast<uint32_t *>(p) + size_t(kReadSlots) * kReadWords, 0,
               size_t(kReadSlots) * kReadBlocks * 4);
-  g_read.ptr = static_cast<uint32_t *>(p);
-  g_read.dev = static_cast<uint32_t *>(d);
-  g_read.seq = 0;
+  st.ptr = static_cast<uint32_t *>(p);
+  st.dev = static_cast<uint32_t *>(d);
+  st.seq = 0;
   return true;
+}
+
+// A stage for this reader, locked: a free one, else its turn at one.
+static ReadStage &take_read_stage(std::unique_lock<std::mutex> &lk) {
+  for (ReadStage &st : g_read) {
+    lk = std::unique_lock<std::mutex>(st.mu, std::try_to_lock);
+    if (lk.owns_lock()) return st;
+  }
+  static std::atomic<uint32_t> turn{0};
+  ReadStage &st = g_read[turn++ % kReadStages];
+  lk = std::unique_lock<std::mutex>(st.mu);
+  return st;
 }
 
 constexpr int kMadvPopulateWrite = 23;  // MADV_POPULATE_WRITE (Linux 5.14)
@@ -208,9 +228,11 @@ constexpr int kMadvPopulateWrite = 23;  // MADV_POPULATE_WRITE (Linux 5.14)
 int read_chunks(uint32_t *out, size_t words, int device, hipStream_t s,
                 const ReadLaunch &launch) {
   if (words == 0) return MK_OK;
-  std::lock_guard<std::mutex> lk(g_read.mu);
+  std::unique_lock<std::mutex> lk;
+  ReadStage &stage = take_read_stage(lk);
   const size_t nchunks = (words + kReadWords - 1) / kReadWords;
-  if (!read_stage_ready()) {  // one device chunk, copied on by the runtime
+  if (!read_stage_ready(stage)) {  // one device chunk, copied on by the runtime
+    lk.unlock();
     DevBuf b;
     if (int r = b.ensure(size_t(kReadWords) * 4)) return r;
     hipError_t e = hipSuccess;
@@ -226,13 +248,13 @@ int read_chunks(uint32_t *out, size_t words, int device, hipStream_t s,
     b.release();
     return e == hipSuccess ? MK_OK : hip_fail(e, "result readback");
   }
-  if (uint64_t(g_read.seq) + nchunks > 0xFFFFFFFFull) {
-    std::memset(g_read.ptr + size_t(kReadSlots) * kReadWords, 0,
+  if (uint64_t(stage.seq) + nchunks > 0xFFFFFFFFull) {
+    std::memset(stage.ptr + size_t(kReadSlots) * kReadWords, 0,
                 size_t(kReadSlots) * kReadBlocks * 4);
-    g_read.seq = 0;
+    stage.seq = 0;
   }
-  const uint32_t seq0 = g_read.seq + 1;
-  g_read.seq += uint32_t(nchunks);
+  const uint32_t seq0 = stage.seq + 1;
+  stage.seq += uint32_t(nchunks);
   // chunks go launched -> arrived (their flags seen) -> taken (by a copying
   // thread) -> copied; chunk c uses slot c % kReadSlots.  Only the calling
   // thread launches and looks at flags; the helpers touch host memory only.
@@ -266,18 +288,37 @@ int read_chunks(uint32_t *out, size_t words, int device, hipStream_t s,
     do {
       if (c >= arrived.load()) return false;
     } while (!taken.compare_exchange_weak(c, c + 1));
-    const uint32_t *buf = g_read.ptr + (c % kReadSlots) * kReadWords;
+    const uint32_t *buf = stage.ptr + (c % kReadSlots) * kReadWords;
     if (!ahead) map_chunk(c);
     std::memcpy(out + c * kReadWords, buf, std::min<size_t>(kReadWords, words - c * kReadWords) * 4);
     copied[c % kReadSlots].store(c + 1);
     return true;
   };
+  // Helpers with nothing to do spin for the time a chunk takes, then sleep
+  // until one arrives (or the read ends).
+  std::mutex sleep_mu;
+  std::condition_variable sleep_cv;
+  std::atomic<uint32_t> asleep{0};
+  auto wake = [&]() {
+    if (asleep.load() == 0) return;
+    { std::lock_guard<std::mutex> sl(sleep_mu); }
+    sleep_cv.notify_all();
+  };
+  auto over = [&]() { return stop.load() || taken.load() >= nchunks; };
   auto help = [&]() {
     uint32_t idle = 0;
-    while (!stop.load() && taken.load() < nchunks) {
-      if (copy_one() || map_one()) idle = 0;
-      else if (++idle < 4096) __builtin_ia32_pause();
-      else std::this_thread::yield();
+    while (!over()) {
+      if (copy_one() || map_one()) {
+        idle = 0;
+      } else if (++idle < 4096) {
+        __builtin_ia32_pause();
+      } else {
+        std::unique_lock<std::mutex> sl(sleep_mu);
+        ++asleep;
+        sleep_cv.wait(sl, [&]() { return over() || taken.load() < arrived.load(); });
+        --asleep;
+        idle = 0;
+      }
     }
   };
   size_t launched = 0;
@@ -287,9 +328,9 @@ int read_chunks(uint32_t *out, size_t words, int device, hipStream_t s,
            (launched < kReadSlots ||
             copied[launched % kReadSlots].load() == launched - kReadSlots + 1)) {
       const size_t slot = launched % kReadSlots;
-      launch(g_read.dev + slot * kReadWords, launched * kReadWords,
+      launch(stage.dev + slot * kReadWords, launched * kReadWords,
              uint32_t(std::min<size_t>(kReadWords, words - launched * kReadWords)),
-             g_read.dev + size_t(kReadSlots) * kReadWords + slot * kReadBlocks,
+             stage.dev + size_t(kReadSlots) * kReadWords + slot * kReadBlocks,
              seq0 + uint32_t(launched));
       e = hipGetLastError();
       if (e == hipSuccess) ++launched;
@@ -310,11 +351,12 @@ int read_chunks(uint32_t *out, size_t words, int device, hipStream_t s,
   bool waited = false;
   while (e == hipSuccess && c < nchunks) {
     launch_more();
-    const volatile uint32_t *flags = g_read.ptr + size_t(kReadSlots) * kReadWords +
+    const volatile uint32_t *flags = stage.ptr + size_t(kReadSlots) * kReadWords +
                                      (c % kReadSlots) * kReadBlocks;
     while (c < launched && block < kReadBlocks && flags[block] == seq0 + uint32_t(c)) ++block;
     if (block == kReadBlocks) {
       arrived.store(++c);
+      wake();
       block = 0;
       spins = 0;
       waited = false;
@@ -334,6 +376,7 @@ int read_chunks(uint32_t *out, size_t words, int device, hipStream_t s,
     stop.store(true);
     (void)hipStreamSynchronize(s);  // no kernel may still write into the slots
   }
+  wake();
   for (unsigned i = 0; i < nh; ++i) helpers[i].join();
   return e == hipSuccess ? MK_OK : hip_fail(e, "result readback");
 }

@@ -7,8 +7,9 @@
 // pinned host memory, in its final form (no device copy of the result), and
 // up to kReadSlots threads, one per slot, copy them on, so that link,
 // copying and the first touch of the caller's pages overlap.  The pinned
-// memory (8 MB) is shared by all handles, one reader at a time; it is
-// allocated by the first read and freed with the last slab pool.
+// memory (8 MB for each of up to kReadStages readers at a time) is shared by
+// all handles; it is allocated by the first reads and freed with the last
+// slab pool.
 #pragma once
 
 #include <functional>
@@ -19,6 +20,7 @@ namespace mk {
 
 constexpr uint32_t kReadWords = 1u << 18;  // words per chunk
 constexpr uint32_t kReadSlots = 8;
+constexpr uint32_t kReadStages = 4;
 constexpr uint32_t kReadBlocks = 32;       // blocks per chunk, a flag word each
 constexpr uint32_t kReadThreads = 1024;
 
