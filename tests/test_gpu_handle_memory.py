@@ -1,6 +1,7 @@
 """Device memory of traversal handles: the arrays of dense steps (6 bytes a
 vertex) belong to the handles that can take such steps."""
 import ctypes
+import gc
 
 import numpy as np
 import pytest
@@ -14,6 +15,7 @@ N = 1 << 22
 
 
 def bytes_of(make):
+    gc.collect()  # what earlier tests left is not freed in between
     torch.cuda.synchronize()
     before = torch.cuda.mem_get_info()[0]
     h = make()

@@ -2,6 +2,7 @@
 than the bound on work items (worked in windows, the count exact), and
 the bound on the static count's scratch, which the fallback gives back."""
 import ctypes
+import gc
 
 import numpy as np
 import pytest
@@ -15,6 +16,7 @@ pytestmark = pytest.mark.gpu
 
 def held(call):
     """Bytes of device memory that `call` leaves allocated."""
+    gc.collect()
     torch.cuda.synchronize()
     before = torch.cuda.mem_get_info()[0]
     call()
